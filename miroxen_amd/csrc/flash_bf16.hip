@@ -149,8 +149,14 @@ __device__ __forceinline__ void load_tile(const uint16_t* src, int t, unsigned c
   constexpr int NOPS = IS_V ? Dims<DH>::VOPS : Dims<DH>::KOPS;
   constexpr int NLD = (NOPS + NW - 1) / NW;
   const int key0 = t * KT;
-  const __amdgpu_buffer_rsrc_t r =
-      buf_rsrc(src + kvbase + int64_t(key0) * p.kv_stride, uint32_t(p.Skv - key0) * uint32_t(p.kv_stride) * 2u);
+  // The resource starts at this head's channels of row key0. D = 64 and 128 read whole
+  // heads, so "rows left times stride" keeps every row past Skv out of it. D = 72 reads
+  // up to 24 channels past its head: for the last head of the last row those lie past the
+  // end of the tensor, so the resource ends with the last row's heads (less than a stride
+  // before, so the rows past Skv stay outside).
+  uint32_t bytes = uint32_t(p.Skv - key0) * uint32_t(p.kv_stride) * 2u;
+  if constexpr (DH % 32 != 0) bytes -= uint32_t(p.kv_stride - (int64_t(p.Hkv) * DH - kvbase)) * 2u;
+  const __amdgpu_buffer_rsrc_t r = buf_rsrc(src + kvbase + int64_t(key0) * p.kv_stride, bytes);
   auto op = [&](auto jjc) __attribute__((always_inline)) {
     constexpr int jj = decltype(jjc)::value;
     if constexpr (NOPS % NW != 0)

@@ -313,6 +313,22 @@ def test_small_head_dim_fast_path(cuda, case):
     _check_guards(buf, 16, Sq, Hq * D, Hq * D, rows)
 
 
+def test_d72_last_head_ends_the_allocation(cuda):
+    """D = 72 reads 16-byte chunks past its 72 channels (to 80 of K, 96 of V). K and V here
+    fill allocations of exactly 18 MiB (nine 2 MiB pages, no slack behind the last head of
+    the last token), so a read past the last head would leave the mapping."""
+    S, H, D = 8192, 16, 72
+    assert S * H * D * 2 == 9 * 2 ** 21
+    print(f"d72 allocation end S={S} H={H}", flush=True)
+    q, k, v, *_ = _make(S, S, H, H, D, 0, 1.0, 72, cuda)
+    p = AttnParams(Sq=64, Skv=S, Hq=H, Hkv=H, D=D)
+    out, _ = _run(flash_attn, q, k, v, p, 64, H * D)
+    rows = [0, 31, 63]
+    want = oracle.attention_f64(_bits(q), _bits(k), _bits(v), 64, S, H, H, D, 0.0, 0, 0,
+                                rows=np.array(rows, np.int32)).reshape(len(rows), -1)
+    assert reference_gate(_f32(out[rows]), want)[0]
+
+
 # Key-range split of the grid's last round (flash_attn_split_plan): the split units'
 # rows against the oracle, parts whose keys are all masked, GQA / D = 64 / 72 with
 # padded strides, and repeat / cross-stream calls sharing the library's split region.
