@@ -96,61 +96,76 @@ __global__ void __launch_bounds__(256) mxfp8_quant(const uint16_t* __restrict__ 
 }
 
 // ---------------- GEMM ----------------
-// One operand's DMA of stage k0: 32 ops of 1 KB (8 rows x 128 B each); wave w
+// One operand's DMA of stage k0: ops of 1 KB (8 rows x 128 B each); wave w of four
 // issues ops j = 4 * jj + w. Lane i of op j fills physical chunk i % 8 of row
 // 8 j + i / 8, i.e. logical chunk (i % 8) ^ ((row >> 1) & 7); ((row >> 1) & 7)
 // depends on j only through its parity, which is the wave's. Both operands have
-// row stride K, so one set of 8 per-lane offsets serves both and the only
+// row stride K, so one set of per-lane offsets serves both and the only
 // scalar offset is k0.
+template <int NV>
 struct OpAddr {
-  uint32_t vo[8];  // row (8 j + lane / 8) * K + logical chunk * 16, j = 4 jj + wave
-  uint32_t chunk;  // logical chunk * 16 (for the K-tail check)
+  uint32_t vo[NV];  // row (8 j + lane / 8) * K + logical chunk * 16, j = 4 jj + wave
+  uint32_t chunk;   // logical chunk * 16 (for the K-tail check)
 };
-__device__ __forceinline__ OpAddr op_addr(int64_t K, int lane, int wave) {
-  OpAddr a;
+template <int NV>
+__device__ __forceinline__ OpAddr<NV> op_addr(int64_t K, int lane, int wave) {
+  OpAddr<NV> a;
   const int rin = lane >> 3, p = lane & 7;
   const int row = 8 * (wave & 1) + rin;  // row modulo 16 is what the swizzle sees
   const int c = p ^ ((row >> 1) & 7);
   a.chunk = uint32_t(c * 16);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) a.vo[jj] = uint32_t(8 * (4 * jj + wave) + rin) * uint32_t(K) + a.chunk;
+  for (int jj = 0; jj < NV; ++jj) a.vo[jj] = uint32_t(8 * (4 * jj + wave) + rin) * uint32_t(K) + a.chunk;
   return a;
 }
-
-// Lanes whose chunk lies past K read zeros (an offset past the buffer's range);
-// for a stage wholly past K every lane does, and the DMA only clears LDS.
-__device__ __forceinline__ void dma_stage(__amdgpu_buffer_rsrc_t rs, const OpAddr& a, int64_t K, int k0,
+// Lanes whose chunk lies past K read zeros (an offset past the buffer's range); for a
+// stage wholly past K every lane does, and the DMA only clears LDS.
+template <int NV>
+__device__ __forceinline__ uint32_t past_k(const OpAddr<NV>& a, int64_t K, int k0) {
+  return uint32_t(k0) + a.chunk >= uint32_t(K) ? 0x80000000u : 0u;
+}
+template <int NV>
+__device__ __forceinline__ void dma_op(__amdgpu_buffer_rsrc_t rs, const OpAddr<NV>& a, int jj, uint32_t past, int k0,
+                                       unsigned char* dst, int wave) {
+  buf2lds16(rs, a.vo[jj] | past, uint32_t(k0), (MXA_LDS void*)(dst + (4 * jj + wave) * 1024));
+}
+template <int NV>
+__device__ __forceinline__ void dma_stage(__amdgpu_buffer_rsrc_t rs, const OpAddr<NV>& a, int64_t K, int k0,
                                           unsigned char* dst, int wave) {
-  const bool past = uint32_t(k0) + a.chunk >= uint32_t(K);
+  const uint32_t past = past_k(a, K, k0);
 #pragma unroll
-  for (int jj = 0; jj < 8; ++jj) {
-    const int j = 4 * jj + wave;
-    const uint32_t off = past ? 0x80000000u : a.vo[jj];
-    buf2lds16(rs, off, uint32_t(k0), (MXA_LDS void*)(dst + j * 1024));
-  }
+  for (int jj = 0; jj < NV; ++jj) dma_op(rs, a, jj, past, k0, dst, wave);
 }
 
-// Epilogue through LDS: the 256 x 256 bf16 Y tile (row m = 512 B of n) fills the
-// stage buffers. Lane (m = lane % 32 of block j, h = lane / 32) holds n = 8g + 4h +
-// (0..3) of block i; 16-byte chunk q of row m sits at q ^ (m % 16), so the 8-byte
-// writes and the 16-byte row reads are free of bank conflicts, and each row goes out
-// as coalesced 16-byte stores. ALPHA: Y = alpha * C (+ Y).
-template <bool ALPHA>
-__device__ __forceinline__ void store_tile(const f32x16 (&acc)[4][4], unsigned char* lds, uint16_t* __restrict__ y,
+// Epilogue through LDS: the TN x TM = 64 NI x 64 NJ bf16 Y tile (row m = 128 NI bytes of
+// n) fills the stage buffers. Lane (m = lane % 32 of block j, h = lane / 32) holds n = 8g
+// + 4h + (0..3) of block i; the 16-byte chunks of row m are XOR'd within groups of 8 or 16
+// so that 16 rows' same chunk covers every bank: the 8-byte writes and the 16-byte row
+// reads are free of bank conflicts, and each row goes out as coalesced 16-byte stores.
+// ALPHA: Y = alpha * C (+ Y).
+template <int NI, int NJ, bool ALPHA>
+__device__ __forceinline__ void store_tile(const f32x16 (&acc)[NI][NJ], unsigned char* lds, uint16_t* __restrict__ y,
                                            int64_t ldy, int M, int N, int m0, int n0, int wm, int wn, int lane,
                                            int beta, float alpha) {
+  constexpr int CH = 8 * NI, RB = 16 * CH;  // chunks and bytes per row
+  auto swz = [](int m) __attribute__((always_inline)) { return NI % 2 == 0 ? m & 15 : (m >> 1) & 7; };
   const int n = lane & 31, h = lane >> 5;
   block_sync();  // every wave is done with the operand buffers
   {
-    const int xs = lane & 15;  // m % 16 (wm and 32 j are multiples of 16)
-    unsigned char* wp = lds + (wm + n) * 512 + 8 * h + wn * 2;
+    const int xs = swz(n);  // wm and 32 j are multiples of 16
+    unsigned char* wp = lds + (wm + n) * RB + 8 * h + wn * 2;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int cs = ((4 * i + g) ^ xs) << 4;
+        // chunk of the row: wn / 8 + 4 i + g. wn is 0 or 32 NI; the XOR stays within the
+        // wave's chunks when 4 NI is a multiple of its span, else it is taken on the whole
+        const int q = 4 * i + g;
+        unsigned char* wq = (4 * NI) % (NI % 2 == 0 ? 16 : 8) == 0
+                                ? wp + ((q ^ xs) << 4)
+                                : lds + (wm + n) * RB + 8 * h + (((wn >> 3) + q) ^ xs) * 16;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NJ; ++j) {
           const f32x16& c = acc[i][j];
           float v[4] = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
           if constexpr (ALPHA) {
@@ -166,18 +181,17 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[4][4], unsigned c
                 if (nb + e < N) v[e] += bf2f(p[e]);
             }
           }
-          *reinterpret_cast<u32x2*>(wp + j * 32 * 512 + cs) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          *reinterpret_cast<u32x2*>(wq + j * 32 * RB) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         }
       }
   }
   block_sync();
   const bool vec = (reinterpret_cast<uintptr_t>(y) & 15) == 0 && ldy % 8 == 0;
-  const int c = threadIdx.x & 31, nn = n0 + 8 * c;
 #pragma unroll 4
-  for (int it = 0; it < 32; ++it) {
-    const int r = it * 8 + (threadIdx.x >> 5), m = m0 + r;
+  for (int it = 0; it < 2 * NJ * NI; ++it) {
+    const int idx = it * 256 + int(threadIdx.x), r = idx / CH, c = idx % CH, m = m0 + r, nn = n0 + 8 * c;
     if (m >= M) break;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * 512 + ((c ^ (r & 15)) << 4));
+    const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * RB + ((c ^ swz(r)) << 4));
     uint16_t* p = y + int64_t(m) * ldy + nn;
     if (vec && nn + 7 < N) {
       *reinterpret_cast<u32x4*>(p) = v;
@@ -189,13 +203,73 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[4][4], unsigned c
   }
 }
 
+// The scale words of NB consecutive 32-row blocks for the four K blocks of one stage, in
+// the reference's 128 x 4 interleaved layout: byte (r / 128) kbp 128 + (kb / 4) 512 +
+// (r % 32) 16 + ((r % 128) / 32) 4 + kb % 4. A 128-row band puts its four row blocks next
+// to each other, so aligned runs of 4 or 2 blocks are one 16- or 8-byte load per lane.
+template <int NB>
+struct ScaleAddr {
+  uint32_t off[NB == 3 ? 3 : 1];
+};
+template <int NB>
+__device__ __forceinline__ ScaleAddr<NB> scale_addr(int row0, int kbp, int n) {
+  ScaleAddr<NB> a;
+#pragma unroll
+  for (int b = 0; b < (NB == 3 ? 3 : 1); ++b) {
+    const int r = row0 + 32 * b;
+    a.off[b] = uint32_t(r / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n) + uint32_t((r % 128) / 32) * 4u;
+  }
+  return a;
+}
+template <int NB>
+__device__ __forceinline__ void scale_load(__amdgpu_buffer_rsrc_t rs, const ScaleAddr<NB>& a, uint32_t soff,
+                                           uint32_t (&w)[NB]) {
+  if constexpr (NB == 4) {
+    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, a.off[0], soff, 0));
+    w[0] = v[0], w[1] = v[1], w[2] = v[2], w[3] = v[3];
+  } else if constexpr (NB == 2) {
+    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, a.off[0], soff, 0));
+    w[0] = v[0], w[1] = v[1];
+  } else {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) w[b] = __builtin_amdgcn_raw_buffer_load_b32(rs, a.off[b], soff, 0);
+  }
+}
+
+// One LDS operand read of 16 bytes: chunk coff of row block blk (32 rows) of a stage.
+__device__ __forceinline__ void op_read(const unsigned char* base, int blk, int coff, int hi, i32x8& d) {
+  const i32x4 v = *reinterpret_cast<const i32x4*>(base + blk * 32 * kStage + coff);
+  if (hi == 0) d = __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1);
+  else d = __builtin_shufflevector(d, __builtin_shufflevector(v, v, 0, 1, 2, 3, 0, 1, 2, 3), 0, 1, 2, 3, 8, 9, 10, 11);
+}
+#define MXA_SCHED __builtin_amdgcn_sched_barrier(0)
+
+// MXFP8 GEMM on tiles of TN = 64 NI n x TM = 64 NJ m; wave (wn, wm) of 2 x 2 owns 32 NI x
+// 32 NJ.
+//
+// What bounds it (8192 x 12288 x 4096, 256 x 256 tiles): a 64-wide K step is NI NJ MFMAs of
+// 64 cycles, so a 128-byte stage cannot take less than 2048 cycles; its LDS-DMA (64 KB)
+// takes 1300 cycles when every line hits L2 and ~2000 with this grid's misses, and four
+// waves that issue more than one DMA op per ~80 cycles each fill the address queue, behind
+// which the wave's next MFMA waits. So the order of a stage is written out instruction by
+// instruction (MXA_SCHED keeps the compiler from regrouping it): one MFMA, then at most one
+// LDS operand read of the next K step and at most one DMA op, DMA ops 1.25 MFMAs apart. The
+// compiler's grouping (all 16 DMA ops within five MFMAs, and scale words unpacked after the
+// first DMA ops, which waited for those to land) took 3150-3270 cycles a stage, this order
+// 2340 (MFMAs and barriers alone: 2245); the chip then runs at its power limit (1.71
+// instead of 2.05 GHz), so the GEMM gains less: 344 -> 310 us on operands resident in the
+// caches; with the prefetch below, 377 -> 318 us on operands that come from HBM.
+template <int NI, int NJ>
 __global__ void __launch_bounds__(256, 1)
 mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, const uint8_t* __restrict__ xq,
            const uint8_t* __restrict__ xsf, uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K, int beta,
            int ntn, int ntm) {
-  __shared__ __align__(16) unsigned char lds[4 * kStageB];
-  // stage buffers: operand A at lds + (st % 2) * kStageB, operand B 64 KB above it
-  unsigned char *const a0 = lds, *const a1 = lds + kStageB, *const b0 = lds + 2 * kStageB;
+  constexpr int TN = 64 * NI, TM = 64 * NJ, SA = TN * kStage, SB = TM * kStage;
+  constexpr int NV = 2 * (NI > NJ ? NI : NJ);
+  // stage buffers: operand W at lds + (st % 2) * SA, operand X at lds + 2 SA + (st % 2) * SB
+  // (one LDS object: with a second one the compiler waits for every DMA before LDS reads)
+  __shared__ __align__(16) unsigned char lds[2 * (SA + SB) + 4 * 256];
+  unsigned char *const a0 = lds, *const a1 = lds + SA, *const b0 = lds + 2 * SA, *const b1 = lds + 2 * SA + SB;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int L = xcd_remap(blockIdx.x, gridDim.x);
@@ -204,34 +278,22 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   // and share 12 operand strips instead of 33
   const int gsz = kGroupM * ntn, grp = L / gsz, fm = grp * kGroupM;
   const int gm = min(ntm - fm, kGroupM), li = L - grp * gsz;
-  const int tm = fm + li % gm, tn = li / gm;
-  const int n0 = tn * kTile, m0 = tm * kTile;
-  const int wn = (wave & 1) * 128, wm = (wave >> 1) * 128;
+  const int tm = li % gm, tn = li / gm;
+  const int n0 = tn * TN, m0 = (fm + tm) * TM;
+  const int wn = (wave & 1) * (32 * NI), wm = (wave >> 1) * (32 * NJ);
   const int kbp = int(pad_up(K / kMxBlock, 4));
   const int nst = (K + kStage - 1) / kStage;
 
   const __amdgpu_buffer_rsrc_t rw = buf_rsrc(wq + int64_t(n0) * K, uint32_t(int64_t(N - n0) * K));
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xq + int64_t(m0) * K, uint32_t(int64_t(M - m0) * K));
-  const OpAddr oa = op_addr(K, lane, wave_u);
-  // Scales, in the reference's 128 x 4 interleaved layout: byte (r / 128) kbp 128 +
-  // (kb / 4) 512 + (r % 32) 16 + ((r % 128) / 32) 4 + kb % 4. A wave's 128 rows are one
-  // 128-row band, so lane n's four row blocks (r % 32 = n, (r % 128) / 32 = b) for the
-  // four K blocks of stage st (kb / 4 = st) are the 16 contiguous bytes at
-  // band + st 512 + 16 n: one 16-byte load per operand per stage. Bands past the
-  // 128-padded matrix read as zeros (their data is zero too).
+  const OpAddr<NV> oa = op_addr<NV>(K, lane, wave_u);
+  // scale words of a stage, loaded a stage ahead; blocks past the 128-padded matrix read as
+  // zeros (their data is zero too)
   const int n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rsw = buf_rsrc(wsf, uint32_t(pad_up(N, 128) * kbp));
   const __amdgpu_buffer_rsrc_t rsx = buf_rsrc(xsf, uint32_t(pad_up(M, 128) * kbp));
-  const uint32_t sw_off = uint32_t((n0 + wn) / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n);
-  const uint32_t sx_off = uint32_t((m0 + wm) / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n);
-  // raw scale words of stage st (word b = row block b), loaded a stage ahead and
-  // unpacked only after the next stage's wait, so no stage waits on their latency
-  auto scales = [&](int st, uint32_t (&ra)[4], uint32_t (&rb)[4]) __attribute__((always_inline)) {
-    const u32x4 wa = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsw, sw_off + uint32_t(st * 512), 0, 0));
-    const u32x4 wb = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsx, sx_off + uint32_t(st * 512), 0, 0));
-#pragma unroll
-    for (int b = 0; b < 4; ++b) ra[b] = wa[b], rb[b] = wb[b];
-  };
+  const ScaleAddr<NI> sw = scale_addr<NI>(n0 + wn, kbp, n);
+  const ScaleAddr<NJ> sx = scale_addr<NJ>(m0 + wm, kbp, n);
 
   // LDS operand reads: rows row0 + n of an operand tile for K step s. In the f8
   // operand of the 32x32x64 MFMA, bytes 0-15 of lane half h are K 16h .. 16h+15 and
@@ -248,127 +310,155 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
     coff[2 * s + 1] = ((4 * s + 2 + h) ^ x) << 4;
   }
   const int abase = (wn + n) * kStage, bbase = (wm + n) * kStage;
-  auto opread = [&](const unsigned char* base, int b, int s) __attribute__((always_inline)) -> i32x8 {
-    const unsigned char* rp = base + b * 32 * kStage;
-    const i32x4 lo = *reinterpret_cast<const i32x4*>(rp + coff[2 * s]);
-    const i32x4 hi = *reinterpret_cast<const i32x4*>(rp + coff[2 * s + 1]);
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  };
 
-  f32x16 acc[4][4];
+  f32x16 acc[NI][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       // opaque zeros: left as constants, the register allocator splits the
       // accumulators' live ranges at the loop header and spills them
       acc[i][j] = f32x16{};
       asm volatile("" : "+a"(acc[i][j]));
     }
 
-  // DMA of stage st (operands and the raw scale words) into buffers (da, db)
-  auto fetch = [&](int st, unsigned char* da, unsigned char* db, uint32_t (&ra)[4],
-                   uint32_t (&rb)[4]) __attribute__((always_inline)) {
-    dma_stage(rw, oa, K, st * kStage, da, wave_u);
-    dma_stage(rx, oa, K, st * kStage, db, wave_u);
-    scales(st, ra, rb);
+  // MFMA slots of a stage: [0, SL) K step 0, [SL, 2 SL) K step 1, the stage barrier before
+  // slot SL + PRE (PRE MFMAs keep the matrix core busy while a wave waits there). DMA op u
+  // of stage st + 2 goes into slot SL + PRE + 5/8 * 2 SL * u / ND of stage st, the last ones
+  // into the first slots of stage st + 1; operand reads run NP pieces ahead.
+  constexpr int SL = NI * NJ, PRE = SL >= 8 ? 2 : 1, ND = 2 * (NI + NJ), NP = 2 * (NI + NJ);
+  auto dma_slot = [](int u) constexpr { return SL + PRE + u * 5 * SL / (4 * ND); };
+  static_assert(PRE + 15 * 5 * SL / (4 * 16) < 2 * SL, "a stage's DMA ends before its wait");
+  // DMA op u: operand u & 1 (X's ops run out first or last when NI != NJ), index u >> 1
+  auto dma = [&](auto uc, int st, uint32_t past, unsigned char* da, unsigned char* db) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value, lo = 2 * (NI < NJ ? NI : NJ);
+    constexpr bool isx = u < 2 * lo ? (u & 1) : NJ > NI;
+    constexpr int jj = u < 2 * lo ? u >> 1 : u - lo;
+    if constexpr (isx) dma_op(rx, oa, jj, past, st * kStage, db, wave_u);
+    else dma_op(rw, oa, jj, past, st * kStage, da, wave_u);
   };
-  // byte 0: K block 2s + h of step s = 0, byte 2: of step s = 1 (op_sel 0 / 2)
-  auto unpack = [&](const uint32_t (&ra)[4], const uint32_t (&rb)[4], uint32_t (&ta)[4],
-                    uint32_t (&tb)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b) ta[b] = (ra[b] >> (8 * h)) & 0x00FF00FFu, tb[b] = (rb[b] >> (8 * h)) & 0x00FF00FFu;
+  // operand read piece u of K step S: blocks in the order a0, b0 .. b(NJ-1), a1 .., two halves each
+  auto rd = [&](auto sc, auto uc, const unsigned char* ca, const unsigned char* cb, i32x8 (&av)[NI],
+                i32x8 (&bv)[NJ]) __attribute__((always_inline)) {
+    constexpr int S = decltype(sc)::value, o = decltype(uc)::value >> 1, hi = decltype(uc)::value & 1;
+    if constexpr (o == 0) op_read(ca + abase, 0, coff[2 * S + hi], hi, av[0]);
+    else if constexpr (o <= NJ) op_read(cb + bbase, o - 1, coff[2 * S + hi], hi, bv[o - 1]);
+    else op_read(ca + abase, o - NJ, coff[2 * S + hi], hi, av[o - NJ]);
   };
-  auto rd = [&](const unsigned char* ca, const unsigned char* cb, auto sc, i32x8 (&av)[4],
-                i32x8 (&bv)[4]) __attribute__((always_inline)) {
-    constexpr int S = decltype(sc)::value;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      av[b] = opread(ca + abase, b, S);
-      bv[b] = opread(cb + bbase, b, S);
-    }
-  };
-  // operands stay in VGPRs (the 256 accumulators fill the AGPR file); the pin
-  // is also where the reads are waited for
-  auto pin = [&](i32x8 (&av)[4], i32x8 (&bv)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b) asm volatile("" : "+v"(av[b]), "+v"(bv[b]));
-  };
-  // MFMAs [lo, hi) of a K step, in (i, j) order
-  auto mm = [&](const i32x8 (&av)[4], const i32x8 (&bv)[4], const uint32_t (&ta)[4], const uint32_t (&tb)[4],
-                auto sc, auto lo, auto hi) __attribute__((always_inline)) {
-    constexpr int S = decltype(sc)::value;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (4 * i + j >= decltype(lo)::value && 4 * i + j < decltype(hi)::value)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av[i], bv[j], acc[i][j], 0, 0, 2 * S,
-                                                                     int(ta[i]), 2 * S, int(tb[j]));
+  // MFMA q of K step S: the UE8M0 byte of K block 2S + h is byte 2S of the scale word
+  // shifted right by 8h
+  auto mm = [&](auto sc, auto qc, const i32x8 (&av)[NI], const i32x8 (&bv)[NJ], const uint32_t (&ta)[NI],
+                const uint32_t (&tb)[NJ]) __attribute__((always_inline)) {
+    constexpr int S = decltype(sc)::value, i = decltype(qc)::value / NJ, j = decltype(qc)::value % NJ;
+    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av[i], bv[j], acc[i][j], 0, 0, 2 * S, int(ta[i]),
+                                                               2 * S, int(tb[j]));
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
 
-  // Software pipeline: the LDS reads of the next K step are in flight while the
-  // current step's 16 MFMAs run. Stage st + 2 is DMA'd into stage st's buffers
-  // once every wave has read them (the barrier after the step-1 reads).
-  uint32_t ra[4], rb[4], ta[4], tb[4];
-  i32x8 r0a[4], r0b[4], r1a[4], r1b[4];
-  fetch(0, a0, b0, ra, rb);
+  uint32_t ra[NI], rb[NJ];                    // raw scale words of the next stage
+  uint32_t ta0[NI], tb0[NJ], ta1[NI], tb1[NJ];  // shifted words by stage parity
+  i32x8 r0a[NI], r0b[NJ], r1a[NI], r1b[NJ];     // operands of K steps 0 and 1
+  auto scales = [&](int st) __attribute__((always_inline)) {
+    scale_load<NI>(rsw, sw, uint32_t(st * 512), ra);
+    scale_load<NJ>(rsx, sx, uint32_t(st * 512), rb);
+  };
+  auto unpack = [&](uint32_t (&ta)[NI], uint32_t (&tb)[NJ]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < NI; ++b) ta[b] = ra[b] >> (8 * h);
+#pragma unroll
+    for (int b = 0; b < NJ; ++b) tb[b] = rb[b] >> (8 * h);
+  };
+  // L2 prefetch: a stage's DMA has one stage to land, less than a miss to HBM takes, so four
+  // bytes of each line of stage st + kAhead are loaded (into LDS that nothing reads) while
+  // stage st runs. The gm work-groups of one XCD that share a W strip touch a gm-th of its
+  // lines each, the neighbours along n a quarter of the X strip. Waves 0-1: W, 2-3: X.
+  // 8192 x 12288 x 4096 with operands that are not in any cache: 360 -> 318 us (resident
+  // operands: no change); touching half a strip each 328, two stages further ahead 320.
+  constexpr int kAhead = 4, kTouchSlot = SL / 2;
+  const __amdgpu_buffer_rsrc_t rt = wave_u < 2 ? rw : rx;
+  const int share = wave_u < 2 ? gm : min(ntn, 4), strip = wave_u < 2 ? TN : TM;
+  const int per = (strip + share - 1) / share, slice = wave_u < 2 ? tm : tn % share;
+  const uint32_t toff = uint32_t(slice * per + ((wave_u & 1) * 64 + lane) * per / 128) * uint32_t(K);
+  auto touch = [&](int st) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (MXA_LDS void*)(lds + 2 * (SA + SB) + wave_u * 256), 4,
+                                             st < nst ? toff : 0x80000000u, uint32_t(st * kStage), 0, 0);
+  };
+  static_assert(dma_slot(ND - 1) - 2 * SL < kTouchSlot, "the touch is the newest load at the stage's wait");
+  for (int st = 1; st < kAhead; ++st) touch(st);
+  dma_stage(rw, oa, K, 0, a0, wave_u);
+  dma_stage(rx, oa, K, 0, b0, wave_u);
+  scales(0);
   wait_vm();
   block_sync();
-  unpack(ra, rb, ta, tb);
-  fetch(1, a1, b0 + kStageB, ra, rb);
-  rd(a0, b0, S0{}, r0a, r0b);
-  pin(r0a, r0b);
+  unpack(ta0, tb0);
+  {
+    const uint32_t past = past_k(oa, K, kStage);
+    static_for<ND>([&](auto u) __attribute__((always_inline)) {  // the late ops of stage 1 are issued in stage 0
+      if constexpr (dma_slot(decltype(u)::value) < 2 * SL) dma(u, 1, past, a1, b1);
+    });
+  }
+  scales(1);
+  static_for<NP>([&](auto u) __attribute__((always_inline)) { rd(S0{}, u, a0, b0, r0a, r0b); });
+  MXA_SCHED;
 
-  using C0 = std::integral_constant<int, 0>;
-  using C2 = std::integral_constant<int, 2>;
-  using C16 = std::integral_constant<int, 16>;
-  // Stage body. Step 0's MFMAs are interleaved with step 1's LDS reads; two of
-  // step 1's MFMAs are issued before the stage barrier so the matrix unit stays
-  // busy while the wave waits there; the remaining 14 are interleaved with the
-  // DMA of stage st + 2 (unconditional: a stage past K only clears LDS that is
-  // never read) and with the LDS reads of the next stage's step 0 (on the last
-  // stage they fetch stale data that is never used).
-  auto stage = [&](int st, unsigned char* ca, unsigned char* cb, const unsigned char* na,
-                   const unsigned char* nb) __attribute__((always_inline)) {
-    rd(ca, cb, S1{}, r1a, r1b);
-    mm(r0a, r0b, ta, tb, S0{}, C0{}, C16{});
+  // Stage st: operands in (ca, cb), stage st + 1 in (na, nb); (ta, tb) its scales, (un, vn)
+  // those of stage st + 1.
+  auto stage = [&](int st, unsigned char* ca, unsigned char* cb, unsigned char* na, unsigned char* nb,
+                   const uint32_t (&ta)[NI], const uint32_t (&tb)[NJ], uint32_t (&un)[NI],
+                   uint32_t (&vn)[NJ]) __attribute__((always_inline)) {
+    const uint32_t late = past_k(oa, K, (st + 1) * kStage), past = past_k(oa, K, (st + 2) * kStage);
+    static_for<SL>([&](auto qc) __attribute__((always_inline)) {
+      constexpr int q = decltype(qc)::value;
+      mm(S0{}, qc, r0a, r0b, ta, tb);
+      static_for<NP>([&](auto u) __attribute__((always_inline)) {
+        if constexpr (decltype(u)::value * SL / NP == q) rd(S1{}, u, ca, cb, r1a, r1b);
+      });
+      static_for<ND>([&](auto u) __attribute__((always_inline)) {
+        if constexpr (dma_slot(decltype(u)::value) - 2 * SL == q) dma(u, st + 1, late, na, nb);
+      });
+      if constexpr (q == kTouchSlot) {
+        MXA_SCHED;
+        touch(st + kAhead);
+      }
+      MXA_SCHED;
+    });
+    static_for<PRE>([&](auto qc) __attribute__((always_inline)) {
+      mm(S1{}, qc, r1a, r1b, ta, tb);
+      MXA_SCHED;
+    });
+    wait_vm_n<1>();  // this wave's DMA of stage st+1 (and its scale words; not the touch) landed ...
+    block_sync();    // ... for every wave, and every wave has read stage st
+    MXA_SCHED;
+    static_for<SL - PRE>([&](auto qc) __attribute__((always_inline)) {
+      constexpr int q = decltype(qc)::value;
+      mm(S1{}, std::integral_constant<int, PRE + q>{}, r1a, r1b, ta, tb);
+      static_for<ND>([&](auto u) __attribute__((always_inline)) {
+        if constexpr (dma_slot(decltype(u)::value) - SL - PRE == q) dma(u, st + 2, past, ca, cb);
+      });
+      static_for<NP>([&](auto u) __attribute__((always_inline)) {
+        if constexpr (decltype(u)::value * (SL - PRE - (SL >= 8 ? 2 : 0)) / NP == q)
+          rd(S0{}, u, na, nb, r0a, r0b);  // on the last stage: stale data, never used
+      });
+      if constexpr (q == 0) {
+        unpack(un, vn);
+        // the words are consumed here, before the next loads into them are issued
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    pin(r1a, r1b);
-    mm(r1a, r1b, ta, tb, S1{}, C0{}, C2{});
-    __builtin_amdgcn_sched_barrier(0);
-    uint32_t tn[4], tm[4];
-    wait_vm();     // this wave's DMA of stage st+1 (and its scale words) landed ...
-    block_sync();  // ... for every wave, and every wave has read stage st
-    unpack(ra, rb, tn, tm);
-    fetch(st + 2, ca, cb, ra, rb);
-    rd(na, nb, S0{}, r0a, r0b);
-    mm(r1a, r1b, ta, tb, S1{}, C2{}, C16{});
+        for (int b = 0; b < NI; ++b) asm volatile("" : "+v"(un[b]));
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);  // VMEM: DMA, scale loads
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // DS read
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    pin(r0a, r0b);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) ta[b] = tn[b], tb[b] = tm[b];
+        for (int b = 0; b < NJ; ++b) asm volatile("" : "+v"(vn[b]));
+      }
+      if constexpr (q == (SL - PRE > 1 ? 1 : 0)) scales(st + 2);
+      MXA_SCHED;
+    });
   };
   for (int st = 0; st < nst; st += 2) {
-    stage(st, a0, b0, a1, b0 + kStageB);
-    if (st + 1 < nst) stage(st + 1, a1, b0 + kStageB, a0, b0);
+    stage(st, a0, b0, a1, b1, ta0, tb0, ta1, tb1);
+    if (st + 1 < nst) stage(st + 1, a1, b1, a0, b0, ta1, tb1, ta0, tb0);
   }
   wait_vm();  // no LDS-DMA may land after the work-group ends
 
-  store_tile<false>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, 1.f);
+  store_tile<NI, NJ, false>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, 1.f);
 }
 
 
@@ -517,7 +607,7 @@ nvfp4_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
 
   const __amdgpu_buffer_rsrc_t rw = buf_rsrc(wq + int64_t(n0) * RB, uint32_t(int64_t(N - n0) * RB));
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xq + int64_t(m0) * RB, uint32_t(int64_t(M - m0) * RB));
-  const OpAddr oa = op_addr(RB, lane, wave_u);
+  const OpAddr<8> oa = op_addr<8>(RB, lane, wave_u);
   // Scales: a wave's 128 rows are one 128-row band; lane n's bytes for row blocks b =
   // 0..3 (r % 32 = n, (r % 128) / 32 = b) and K blocks 4t..4t+3 are the 16 bytes at
   // band + t 512 + 16 n (word b, byte kb % 4). A stage's 16 blocks: 4 loads per operand.
@@ -593,7 +683,7 @@ nvfp4_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   wait_vm();  // no LDS-DMA may land after the work-group ends
   const float aw = *wamax, ax = *xamax;
   const float alpha = (aw > 0.f ? aw / kFp4Range : 1.f) * (ax > 0.f ? ax / kFp4Range : 1.f);
-  store_tile<true>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, alpha);
+  store_tile<4, 4, true>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, alpha);
 }
 
 }  // namespace
@@ -616,7 +706,7 @@ hipError_t launch_mxfp8_gemm(const uint8_t* wq, const uint8_t* wsf, const uint8_
   const int ntn = (N + kTile - 1) / kTile, ntm = (M + kTile - 1) / kTile;
   const int64_t blocks = int64_t(ntn) * ntm;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(mxfp8_gemm, dim3(unsigned(blocks)), dim3(256), 0, s, wq, wsf, xq, xsf, y, ldy, M, N, K, beta,
+  hipLaunchKernelGGL((mxfp8_gemm<4, 4>), dim3(unsigned(blocks)), dim3(256), 0, s, wq, wsf, xq, xsf, y, ldy, M, N, K, beta,
                      ntn, ntm);
   return hipGetLastError();
 }
