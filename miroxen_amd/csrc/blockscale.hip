@@ -359,9 +359,12 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   uint32_t ra[NI], rb[NJ];                    // raw scale words of the next stage
   uint32_t ta0[NI], tb0[NJ], ta1[NI], tb1[NJ];  // shifted words by stage parity
   i32x8 r0a[NI], r0b[NJ], r1a[NI], r1b[NJ];     // operands of K steps 0 and 1
+  // (past the last stage: the last one's words again, never used; the stage is a scalar
+  // offset, which the buffer's range check need not cover)
   auto scales = [&](int st) __attribute__((always_inline)) {
-    scale_load<NI>(rsw, sw, uint32_t(st * 512), ra);
-    scale_load<NJ>(rsx, sx, uint32_t(st * 512), rb);
+    const uint32_t so = uint32_t(min(st, nst - 1) * 512);
+    scale_load<NI>(rsw, sw, so, ra);
+    scale_load<NJ>(rsx, sx, so, rb);
   };
   auto unpack = [&](uint32_t (&ta)[NI], uint32_t (&tb)[NJ]) __attribute__((always_inline)) {
 #pragma unroll
