@@ -15,7 +15,7 @@
 // The quantizer writes 127 (= 1.0) into every padding byte, so padded K blocks and
 // rows contribute 0 (data 0 times a finite scale) instead of 0 x NaN (0xFF).
 //
-// GEMM (Y[M,N] bf16 = X[M,K] W[N,K]^T, both K-major): tiles of 256 n x 256 m per
+// GEMM (Y[M,N] bf16 = X[M,K] W[N,K]^T, both K-major): the largest tiles are 256 n x 256 m per
 // 4-wave work-group, one wave per SIMD, each wave 128 n x 128 m = 4 x 4 MFMA blocks
 // of 32 x 32 (C = W X^T: lane = one m column, 16 n rows; the 256 fp32 accumulators
 // live in AGPRs). K advances in stages of 128 bytes DMA'd into LDS
@@ -259,17 +259,19 @@ __device__ __forceinline__ void op_read(const unsigned char* base, int blk, int 
 // 2340 (MFMAs and barriers alone: 2245); the chip then runs at its power limit (1.71
 // instead of 2.05 GHz), so the GEMM gains less: 344 -> 310 us on operands resident in the
 // caches; with the prefetch below, 377 -> 318 us on operands that come from HBM.
-template <int NI, int NJ>
+template <int NI, int NJ, int NBUF>
 __global__ void __launch_bounds__(256, 1)
 mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, const uint8_t* __restrict__ xq,
            const uint8_t* __restrict__ xsf, uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K, int beta,
            int ntn, int ntm) {
   constexpr int TN = 64 * NI, TM = 64 * NJ, SA = TN * kStage, SB = TM * kStage;
   constexpr int NV = 2 * (NI > NJ ? NI : NJ);
-  // stage buffers: operand W at lds + (st % 2) * SA, operand X at lds + 2 SA + (st % 2) * SB
+  constexpr bool TOUCH = NBUF == 2;  // L2 prefetch (below)
+  // stage buffers: operand W at lds + (st % NBUF) * SA, operand X behind W's
   // (one LDS object: with a second one the compiler waits for every DMA before LDS reads)
-  __shared__ __align__(16) unsigned char lds[2 * (SA + SB) + 4 * 256];
-  unsigned char *const a0 = lds, *const a1 = lds + SA, *const b0 = lds + 2 * SA, *const b1 = lds + 2 * SA + SB;
+  __shared__ __align__(16) unsigned char lds[NBUF * (SA + SB) + (TOUCH ? 4 * 256 : 0)];
+  auto abuf = [&](int s) __attribute__((always_inline)) { return lds + s * SA; };
+  auto bbuf = [&](int s) __attribute__((always_inline)) { return lds + NBUF * SA + s * SB; };
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int L = xcd_remap(blockIdx.x, gridDim.x);
@@ -323,12 +325,13 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
     }
 
   // MFMA slots of a stage: [0, SL) K step 0, [SL, 2 SL) K step 1, the stage barrier before
-  // slot SL + PRE (PRE MFMAs keep the matrix core busy while a wave waits there). DMA op u
-  // of stage st + 2 goes into slot SL + PRE + 5/8 * 2 SL * u / ND of stage st, the last ones
-  // into the first slots of stage st + 1; operand reads run NP pieces ahead.
+  // slot SL + PRE (PRE MFMAs keep the matrix core busy while a wave waits there). From there
+  // on stage st's buffer is free and takes stage st + NBUF: its DMA op u goes into slot SL +
+  // PRE + 5/8 * 2 SL * u / ND, the last ones into the first slots of stage st + 1.
   constexpr int SL = NI * NJ, PRE = SL >= 8 ? 2 : 1, ND = 2 * (NI + NJ), NP = 2 * (NI + NJ);
+  constexpr int SCL = (NI == 3 ? 3 : 1) + (NJ == 3 ? 3 : 1);  // scale loads per stage
   auto dma_slot = [](int u) constexpr { return SL + PRE + u * 5 * SL / (4 * ND); };
-  static_assert(PRE + 15 * 5 * SL / (4 * 16) < 2 * SL, "a stage's DMA ends before its wait");
+  static_assert(dma_slot(ND - 1) < 3 * SL, "a stage's DMA ends before its wait");
   // DMA op u: operand u & 1 (X's ops run out first or last when NI != NJ), index u >> 1
   auto dma = [&](auto uc, int st, uint32_t past, unsigned char* da, unsigned char* db) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value, lo = 2 * (NI < NJ ? NI : NJ);
@@ -356,109 +359,128 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
 
-  uint32_t ra[NI], rb[NJ];                    // raw scale words of the next stage
-  uint32_t ta0[NI], tb0[NJ], ta1[NI], tb1[NJ];  // shifted words by stage parity
-  i32x8 r0a[NI], r0b[NJ], r1a[NI], r1b[NJ];     // operands of K steps 0 and 1
+  constexpr int NR = NBUF == 2 ? 1 : NBUF;       // sets of raw scale words in flight
+  uint32_t ra[NR][NI], rb[NR][NJ];               // by stage
+  uint32_t ta[NBUF][NI], tb[NBUF][NJ];           // shifted words by stage
+  i32x8 r0a[NI], r0b[NJ], r1a[NI], r1b[NJ];      // operands of K steps 0 and 1
   // (past the last stage: the last one's words again, never used; the stage is a scalar
   // offset, which the buffer's range check need not cover)
-  auto scales = [&](int st) __attribute__((always_inline)) {
+  auto scales = [&](int st, uint32_t (&a)[NI], uint32_t (&b)[NJ]) __attribute__((always_inline)) {
     const uint32_t so = uint32_t(min(st, nst - 1) * 512);
-    scale_load<NI>(rsw, sw, so, ra);
-    scale_load<NJ>(rsx, sx, so, rb);
+    scale_load<NI>(rsw, sw, so, a);
+    scale_load<NJ>(rsx, sx, so, b);
   };
-  auto unpack = [&](uint32_t (&ta)[NI], uint32_t (&tb)[NJ]) __attribute__((always_inline)) {
+  // the words are consumed here, before the next loads into their registers are issued
+  auto unpack = [&](const uint32_t (&a)[NI], const uint32_t (&b)[NJ], uint32_t (&u)[NI],
+                    uint32_t (&v)[NJ]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < NI; ++b) ta[b] = ra[b] >> (8 * h);
+    for (int i = 0; i < NI; ++i) {
+      u[i] = a[i] >> (8 * h);
+      asm volatile("" : "+v"(u[i]));
+    }
 #pragma unroll
-    for (int b = 0; b < NJ; ++b) tb[b] = rb[b] >> (8 * h);
+    for (int j = 0; j < NJ; ++j) {
+      v[j] = b[j] >> (8 * h);
+      asm volatile("" : "+v"(v[j]));
+    }
   };
-  // L2 prefetch: a stage's DMA has one stage to land, less than a miss to HBM takes, so four
-  // bytes of each line of stage st + kAhead are loaded (into LDS that nothing reads) while
-  // stage st runs. The gm work-groups of one XCD that share a W strip touch a gm-th of its
-  // lines each, the neighbours along n a quarter of the X strip. Waves 0-1: W, 2-3: X.
-  // 8192 x 12288 x 4096 with operands that are not in any cache: 360 -> 318 us (resident
-  // operands: no change); touching half a strip each 328, two stages further ahead 320.
+  // L2 prefetch: with two buffers a stage's DMA has one stage to land, less than a miss to
+  // HBM takes, so four bytes of each line of stage st + kAhead are loaded (into LDS that
+  // nothing reads) while stage st runs. The gm work-groups of one XCD that share a W strip
+  // touch a gm-th of its lines each, the neighbours along n a quarter of the X strip. Waves
+  // 0-1: W, 2-3: X. 8192 x 12288 x 4096 with operands that are not in any cache: 360 -> 318
+  // us (resident operands: no change); touching half a strip each 328, two stages further
+  // ahead 320.
   constexpr int kAhead = 4, kTouchSlot = SL / 2;
   const __amdgpu_buffer_rsrc_t rt = wave_u < 2 ? rw : rx;
   const int share = wave_u < 2 ? gm : min(ntn, 4), strip = wave_u < 2 ? TN : TM;
   const int per = (strip + share - 1) / share, slice = wave_u < 2 ? tm : tn % share;
   const uint32_t toff = uint32_t(slice * per + ((wave_u & 1) * 64 + lane) * per / 128) * uint32_t(K);
   auto touch = [&](int st) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (MXA_LDS void*)(lds + 2 * (SA + SB) + wave_u * 256), 4,
-                                             st < nst ? toff : 0x80000000u, uint32_t(st * kStage), 0, 0);
+    if constexpr (TOUCH)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (MXA_LDS void*)(lds + NBUF * (SA + SB) + wave_u * 256), 4,
+                                               st < nst ? toff : 0x80000000u, uint32_t(st < nst ? st * kStage : 0), 0, 0);
   };
-  static_assert(dma_slot(ND - 1) - 2 * SL < kTouchSlot, "the touch is the newest load at the stage's wait");
+  static_assert(!TOUCH || dma_slot(ND - 1) - 2 * SL < kTouchSlot, "the touch is the newest load at the stage's wait");
   for (int st = 1; st < kAhead; ++st) touch(st);
-  dma_stage(rw, oa, K, 0, a0, wave_u);
-  dma_stage(rx, oa, K, 0, b0, wave_u);
-  scales(0);
-  wait_vm();
-  block_sync();
-  unpack(ta0, tb0);
-  {
-    const uint32_t past = past_k(oa, K, kStage);
-    static_for<ND>([&](auto u) __attribute__((always_inline)) {  // the late ops of stage 1 are issued in stage 0
-      if constexpr (dma_slot(decltype(u)::value) < 2 * SL) dma(u, 1, past, a1, b1);
+  constexpr int kEarly = [=] {  // DMA ops of a stage before the next one starts
+    int n = 0;
+    for (int u = 0; u < ND; ++u) n += dma_slot(u) < 2 * SL;
+    return n;
+  }();
+  static_for<NBUF>([&](auto ic) __attribute__((always_inline)) {
+    constexpr int i = decltype(ic)::value;
+    const uint32_t past = past_k(oa, K, i * kStage);
+    static_for<ND>([&](auto u) __attribute__((always_inline)) {  // the late ops of the last one are issued in stage 0
+      if constexpr (i < NBUF - 1 || decltype(u)::value < kEarly) dma(u, i, past, abuf(i), bbuf(i));
     });
+    if constexpr (NR > 1) scales(i, ra[i % NR], rb[i % NR]);
+    else if constexpr (i == 0) scales(0, ra[0], rb[0]);
+    MXA_SCHED;
+    if constexpr (NBUF == 2 && i == 0) {
+      wait_vm();
+      unpack(ra[0], rb[0], ta[0], tb[0]);
+      scales(1, ra[0], rb[0]);
+    }
+  });
+  if constexpr (NBUF > 2) {
+    wait_vm_n<(NBUF - 2) * (ND + SCL) + kEarly + SCL>();
+    unpack(ra[0], rb[0], ta[0], tb[0]);
   }
-  scales(1);
-  static_for<NP>([&](auto u) __attribute__((always_inline)) { rd(S0{}, u, a0, b0, r0a, r0b); });
+  block_sync();
+  static_for<NP>([&](auto u) __attribute__((always_inline)) { rd(S0{}, u, abuf(0), bbuf(0), r0a, r0b); });
   MXA_SCHED;
 
-  // Stage st: operands in (ca, cb), stage st + 1 in (na, nb); (ta, tb) its scales, (un, vn)
-  // those of stage st + 1.
-  auto stage = [&](int st, unsigned char* ca, unsigned char* cb, unsigned char* na, unsigned char* nb,
-                   const uint32_t (&ta)[NI], const uint32_t (&tb)[NJ], uint32_t (&un)[NI],
-                   uint32_t (&vn)[NJ]) __attribute__((always_inline)) {
-    const uint32_t late = past_k(oa, K, (st + 1) * kStage), past = past_k(oa, K, (st + 2) * kStage);
+  // Stage st in buffer s (compile-time).
+  auto stage = [&](int st, auto sc) __attribute__((always_inline)) {
+    constexpr int s = decltype(sc)::value, sn = (s + 1) % NBUF, sp = (s + NBUF - 1) % NBUF;
+    const uint32_t late = past_k(oa, K, (st + NBUF - 1) * kStage), past = past_k(oa, K, (st + NBUF) * kStage);
     static_for<SL>([&](auto qc) __attribute__((always_inline)) {
       constexpr int q = decltype(qc)::value;
-      mm(S0{}, qc, r0a, r0b, ta, tb);
+      mm(S0{}, qc, r0a, r0b, ta[s], tb[s]);
       static_for<NP>([&](auto u) __attribute__((always_inline)) {
-        if constexpr (decltype(u)::value * SL / NP == q) rd(S1{}, u, ca, cb, r1a, r1b);
+        if constexpr (decltype(u)::value * SL / NP == q) rd(S1{}, u, abuf(s), bbuf(s), r1a, r1b);
       });
       static_for<ND>([&](auto u) __attribute__((always_inline)) {
-        if constexpr (dma_slot(decltype(u)::value) - 2 * SL == q) dma(u, st + 1, late, na, nb);
+        if constexpr (dma_slot(decltype(u)::value) - 2 * SL == q) dma(u, st + NBUF - 1, late, abuf(sp), bbuf(sp));
       });
-      if constexpr (q == kTouchSlot) {
+      if constexpr (TOUCH && q == kTouchSlot) {
         MXA_SCHED;
         touch(st + kAhead);
       }
       MXA_SCHED;
     });
     static_for<PRE>([&](auto qc) __attribute__((always_inline)) {
-      mm(S1{}, qc, r1a, r1b, ta, tb);
+      mm(S1{}, qc, r1a, r1b, ta[s], tb[s]);
       MXA_SCHED;
     });
-    wait_vm_n<1>();  // this wave's DMA of stage st+1 (and its scale words; not the touch) landed ...
-    block_sync();    // ... for every wave, and every wave has read stage st
+    // this wave's loads of stage st + 1 landed (newer: the stages up to st + NBUF - 1, touches) ...
+    wait_vm_n<(NBUF - 2) * (ND + SCL + TOUCH) + TOUCH>();
+    block_sync();  // ... for every wave, and every wave has read stage st
     MXA_SCHED;
     static_for<SL - PRE>([&](auto qc) __attribute__((always_inline)) {
       constexpr int q = decltype(qc)::value;
-      mm(S1{}, std::integral_constant<int, PRE + q>{}, r1a, r1b, ta, tb);
+      mm(S1{}, std::integral_constant<int, PRE + q>{}, r1a, r1b, ta[s], tb[s]);
       static_for<ND>([&](auto u) __attribute__((always_inline)) {
-        if constexpr (dma_slot(decltype(u)::value) - SL - PRE == q) dma(u, st + 2, past, ca, cb);
+        if constexpr (dma_slot(decltype(u)::value) - SL - PRE == q) dma(u, st + NBUF, past, abuf(s), bbuf(s));
       });
       static_for<NP>([&](auto u) __attribute__((always_inline)) {
         if constexpr (decltype(u)::value * (SL - PRE - (SL >= 8 ? 2 : 0)) / NP == q)
-          rd(S0{}, u, na, nb, r0a, r0b);  // on the last stage: stale data, never used
+          rd(S0{}, u, abuf(sn), bbuf(sn), r0a, r0b);  // on the last stage: stale data, never used
       });
-      if constexpr (q == 0) {
-        unpack(un, vn);
-        // the words are consumed here, before the next loads into them are issued
-#pragma unroll
-        for (int b = 0; b < NI; ++b) asm volatile("" : "+v"(un[b]));
-#pragma unroll
-        for (int b = 0; b < NJ; ++b) asm volatile("" : "+v"(vn[b]));
-      }
-      if constexpr (q == (SL - PRE > 1 ? 1 : 0)) scales(st + 2);
+      if constexpr (q == 0) unpack(ra[sn % NR], rb[sn % NR], ta[sn], tb[sn]);
+      if constexpr (q == (SL - PRE > 1 ? 1 : 0)) scales(st + NBUF, ra[s % NR], rb[s % NR]);
       MXA_SCHED;
     });
   };
-  for (int st = 0; st < nst; st += 2) {
-    stage(st, a0, b0, a1, b1, ta0, tb0, ta1, tb1);
-    if (st + 1 < nst) stage(st + 1, a1, b1, a0, b0, ta1, tb1, ta0, tb0);
-  }
+  // whole turns of the ring, then the rest (a loop with an exit inside a group would make
+  // the compiler wait for the youngest scale words on every turn)
+  int st = 0;
+  for (; st + NBUF <= nst; st += NBUF)
+    static_for<NBUF>([&](auto s) __attribute__((always_inline)) { stage(st + decltype(s)::value, s); });
+  static_for<NBUF - 1>([&](auto s) __attribute__((always_inline)) {
+    if (st + decltype(s)::value < nst) stage(st + decltype(s)::value, s);
+  });
   wait_vm();  // no LDS-DMA may land after the work-group ends
 
   store_tile<NI, NJ, false>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, 1.f);
@@ -590,6 +612,15 @@ __device__ __forceinline__ f16x8 fp4x8_to_f16(uint32_t d, f16x2 s) {
   return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], e[0], e[1]};
 }
 
+// A block scale (the low byte) in f16, both halves of the pair.
+__device__ __forceinline__ f16x2 fp4_scale(uint32_t byte) {
+  const float f = __builtin_amdgcn_cvt_f32_fp8(int(byte), 0);
+  return __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f, f));
+}
+__device__ __forceinline__ float fp4_alpha(float aw, float ax) {
+  return (aw > 0.f ? aw / kFp4Range : 1.f) * (ax > 0.f ? ax / kFp4Range : 1.f);
+}
+
 __global__ void __launch_bounds__(256, 1)
 nvfp4_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, const float* __restrict__ wamax,
            const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xsf, const float* __restrict__ xamax,
@@ -634,9 +665,7 @@ nvfp4_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   const int abase = (wn + n) * kStage + 8 * h, bbase = (wm + n) * kStage + 8 * h;
   // the block scale of (row block b, chunk c) in f16, both halves of the pair
   auto scale_of = [&](const u32x4 (&sw)[4], int b, int c) __attribute__((always_inline)) -> f16x2 {
-    const uint32_t byte = (sw[c >> 1][b] >> (8 * (2 * (c & 1) + h))) & 0xffu;
-    const float f = __builtin_amdgcn_cvt_f32_fp8(int(byte), 0);
-    return __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f, f));
+    return fp4_scale(sw[c >> 1][b] >> (8 * (2 * (c & 1) + h)));
   };
 
   f32x16 acc[4][4];
@@ -684,9 +713,217 @@ nvfp4_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
     }
   }
   wait_vm();  // no LDS-DMA may land after the work-group ends
-  const float aw = *wamax, ax = *xamax;
-  const float alpha = (aw > 0.f ? aw / kFp4Range : 1.f) * (ax > 0.f ? ax / kFp4Range : 1.f);
+  const float alpha = fp4_alpha(*wamax, *xamax);
   store_tile<4, 4, true>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, alpha);
+}
+
+// ---------------- GEMM of few tiles: K split over the waves of a work-group ----------------
+//
+// A GEMM whose 64- or 128-row tiles leave CUs idle is bound by latency: one work-group
+// walks K in series (M 256, N 3072, K 3072 on 12 tiles of 256 x 256: 24 stages, 34 us; 192
+// tiles of 64 x 64 here: 9.2 us; M 1, N = K = 12288: 128 -> 35 us, 4.3 TB/s of W).
+// Here a work-group of KS waves computes one small tile of TN = 32 NI x TM = 32 NJ and
+// wave w takes the K stages w, w + KS, ..: every wave streams its own 128-byte K slices of
+// the tile's rows into its own ring of NB stage buffers (LDS-DMA, no work-group barrier
+// in the loop, only counted waits), so KS NB stages are in flight per work-group. The fp32
+// partial tiles are added in wave order through LDS (no partial leaves the CU, the sum's
+// order is fixed) and the sum is rounded once.
+//
+// F4: NVFP4. A lane half h reads the 16 bytes of chunk 2 c + h (32 values: two 16-value
+// blocks, K blocks 4 c + 2 h + u) of its row, so the two halves of an f16 MFMA step hold
+// different blocks; W and X use the same assignment and the MFMA sums its K values in any
+// order. Otherwise MXFP8, with the operand layout of mxfp8_gemm.
+template <bool F4, int NI, int NJ, int KS, int NB>
+__global__ void __launch_bounds__(64 * KS, 1)
+gemm_ksplit(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, const float* __restrict__ wamax,
+            const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xsf, const float* __restrict__ xamax,
+            uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K, int beta, int ntm) {
+  constexpr int TN = 32 * NI, TM = 32 * NJ, SA = TN * kStage, ST = (TN + TM) * kStage;
+  constexpr int NSC = F4 ? 4 : 1;                       // scale words per row block and stage
+  constexpr int OPS = 4 * (NI + NJ) + 2 * NSC;          // vector-memory operations per stage
+  constexpr int RED = NI * NJ * 4096;                   // bytes of one wave's partial tile
+  static_assert((NB - 1) * OPS < 64, "the wait counter has 6 bits");
+  __shared__ __align__(16) unsigned char lds[KS * NB * ST > KS * RED ? KS * NB * ST : KS * RED];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, h = lane >> 5;
+  // consecutive tiles share a W strip: the m tiles of one strip run on one XCD
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int n0 = L / ntm * TN, m0 = L % ntm * TM;
+  const int RB = F4 ? K / 2 : K;                        // bytes per row
+  const int kbp = int(pad_up(K / (F4 ? kFp4Block : kMxBlock), 4));
+  const int nst = (RB + kStage - 1) / kStage;
+  const __amdgpu_buffer_rsrc_t rw = buf_rsrc(wq + int64_t(n0) * RB, uint32_t(int64_t(N - n0) * RB));
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xq + int64_t(m0) * RB, uint32_t(int64_t(M - m0) * RB));
+  const __amdgpu_buffer_rsrc_t rsw = buf_rsrc(wsf, uint32_t(pad_up(N, 128) * kbp));
+  const __amdgpu_buffer_rsrc_t rsx = buf_rsrc(xsf, uint32_t(pad_up(M, 128) * kbp));
+  const ScaleAddr<NI> sw = scale_addr<NI>(n0, kbp, n);
+  const ScaleAddr<NJ> sx = scale_addr<NJ>(m0, kbp, n);
+  // DMA op j (rows 8 j .. 8 j + 7): lane i fills physical chunk i % 8 of row 8 j + i / 8,
+  // logical chunk (i % 8) ^ ((row >> 1) & 7), which depends on j through its parity
+  constexpr int NV = 4 * (NI > NJ ? NI : NJ);
+  const int c0 = (lane & 7) ^ (lane >> 4);
+  uint32_t vo[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) vo[j] = uint32_t(8 * j + (lane >> 3)) * uint32_t(RB) + uint32_t((c0 ^ (4 * (j & 1))) * 16);
+  unsigned char* const ring = lds + wave * NB * ST;
+  uint32_t ra[NB][NSC][NI], rb[NB][NSC][NJ];
+  // stage i of this wave (K stage wave + KS i; past the end: zeros, no traffic) into slot s
+  auto issue = [&](int i, auto sc) __attribute__((always_inline)) {
+    constexpr int s = decltype(sc)::value;
+    const int st = wave + KS * i, k0 = st * kStage;
+    const uint32_t p0 = uint32_t(k0 + c0 * 16) >= uint32_t(RB) ? 0x80000000u : 0u;
+    const uint32_t p1 = uint32_t(k0 + (c0 ^ 4) * 16) >= uint32_t(RB) ? 0x80000000u : 0u;
+    unsigned char* d = ring + s * ST;
+#pragma unroll
+    for (int j = 0; j < 4 * NI; ++j) buf2lds16(rw, vo[j] | (j & 1 ? p1 : p0), uint32_t(k0), (MXA_LDS void*)(d + j * 1024));
+#pragma unroll
+    for (int j = 0; j < 4 * NJ; ++j)
+      buf2lds16(rx, vo[j] | (j & 1 ? p1 : p0), uint32_t(k0), (MXA_LDS void*)(d + SA + j * 1024));
+#pragma unroll
+    for (int t = 0; t < NSC; ++t) {
+      // (past the end: the last words again, their data is zero)
+      const uint32_t so = uint32_t(min(st * NSC + t, kbp / 4 - 1) * 512);
+      scale_load<NI>(rsw, sw, so, ra[s][t]);
+      scale_load<NJ>(rsx, sx, so, rb[s][t]);
+    }
+    MXA_SCHED;
+  };
+  f32x16 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x16{};
+
+  const int x = (n >> 1) & 7;
+  const int cnt = (nst - wave + KS - 1) / KS;  // this wave's stages (wave < KS; may be 0)
+  static_for<NB>([&](auto s) __attribute__((always_inline)) { issue(decltype(s)::value, s); });
+  auto body = [&](int i, auto sc) __attribute__((always_inline)) {
+    constexpr int s = decltype(sc)::value;
+    wait_vm_n<(NB - 1) * OPS>();
+    const unsigned char* d = ring + s * ST + n * kStage;
+    // this half's 16-byte chunks of a row: 2 r + h
+    i32x4 av[NI][4], bv[NJ][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int co = ((2 * r + h) ^ x) << 4;
+#pragma unroll
+      for (int b = 0; b < NI; ++b) av[b][r] = *reinterpret_cast<const i32x4*>(d + b * 32 * kStage + co);
+#pragma unroll
+      for (int b = 0; b < NJ; ++b) bv[b][r] = *reinterpret_cast<const i32x4*>(d + SA + b * 32 * kStage + co);
+    }
+    uint32_t ta[NSC][NI], tb[NSC][NJ];
+#pragma unroll
+    for (int t = 0; t < NSC; ++t) {
+#pragma unroll
+      for (int b = 0; b < NI; ++b) ta[t][b] = ra[s][t][b] >> ((F4 ? 16 : 8) * h);
+#pragma unroll
+      for (int b = 0; b < NJ; ++b) tb[t][b] = rb[s][t][b] >> ((F4 ? 16 : 8) * h);
+    }
+    // every operand read has returned and the scale words are consumed before the slot is refilled
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int b = 0; b < NI; ++b) asm volatile("" : "+v"(av[b][r]));
+#pragma unroll
+      for (int b = 0; b < NJ; ++b) asm volatile("" : "+v"(bv[b][r]));
+    }
+#pragma unroll
+    for (int t = 0; t < NSC; ++t) {
+#pragma unroll
+      for (int b = 0; b < NI; ++b) asm volatile("" : "+v"(ta[t][b]));
+#pragma unroll
+      for (int b = 0; b < NJ; ++b) asm volatile("" : "+v"(tb[t][b]));
+    }
+    issue(i + NB, sc);  // (ends with a scheduling barrier)
+    if constexpr (!F4) {
+      static_for<2>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value;
+#pragma unroll
+        for (int i2 = 0; i2 < NI; ++i2)
+#pragma unroll
+          for (int j2 = 0; j2 < NJ; ++j2)
+            acc[i2][j2] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                __builtin_shufflevector(av[i2][2 * k], av[i2][2 * k + 1], 0, 1, 2, 3, 4, 5, 6, 7),
+                __builtin_shufflevector(bv[j2][2 * k], bv[j2][2 * k + 1], 0, 1, 2, 3, 4, 5, 6, 7), acc[i2][j2], 0, 0,
+                2 * k, int(ta[0][i2]), 2 * k, int(tb[0][j2]));
+      });
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f16x2 pa[NI], pb[NJ];
+#pragma unroll
+          for (int b = 0; b < NI; ++b) pa[b] = fp4_scale(ta[r][b] >> (8 * u));
+#pragma unroll
+          for (int b = 0; b < NJ; ++b) pb[b] = fp4_scale(tb[r][b] >> (8 * u));
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            f16x8 fa[NI], fb[NJ];
+#pragma unroll
+            for (int b = 0; b < NI; ++b) fa[b] = fp4x8_to_f16(uint32_t(av[b][r][2 * u + w]), pa[b]);
+#pragma unroll
+            for (int b = 0; b < NJ; ++b) fb[b] = fp4x8_to_f16(uint32_t(bv[b][r][2 * u + w]), pb[b]);
+#pragma unroll
+            for (int i2 = 0; i2 < NI; ++i2)
+#pragma unroll
+              for (int j2 = 0; j2 < NJ; ++j2)
+                acc[i2][j2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i2], fb[j2], acc[i2][j2], 0, 0, 0);
+          }
+        }
+    }
+    MXA_SCHED;
+  };
+  // whole turns of the ring, then the rest (see mxfp8_gemm)
+  int i = 0;
+  for (; i + NB <= cnt; i += NB)
+    static_for<NB>([&](auto s) __attribute__((always_inline)) { body(i + decltype(s)::value, s); });
+  static_for<NB - 1>([&](auto s) __attribute__((always_inline)) {
+    if (i + decltype(s)::value < cnt) body(i + decltype(s)::value, s);
+  });
+  wait_vm();        // no LDS-DMA may land in what the reduction writes
+  __syncthreads();  // every wave is done with the rings
+
+  // Reduction: [wave][block][g = 4 rows of n][2 halves][32 m] groups of four n in fp32, the m
+  // slot XOR'd with the group's position along n so that reads along n are conflict-free.
+  float alpha = 1.f;
+  if constexpr (F4) alpha = fp4_alpha(*wamax, *xamax);
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int sl = n ^ (2 * g + h + 8 * (i & 1));
+        *reinterpret_cast<f32x4*>(lds + wave * RED + (((i * NJ + j) * 4 + g) * 64 + h * 32 + sl) * 16) =
+            f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+      }
+  __syncthreads();
+  const bool vec = (reinterpret_cast<uintptr_t>(y) & 7) == 0 && ldy % 4 == 0;
+  constexpr int Q = TN / 4;  // groups of four n per row
+  for (int t = threadIdx.x; t < Q * TM; t += 64 * KS) {
+    const int q = t % Q, ml = t / Q, i = q >> 3, g = (q >> 1) & 3, hh = q & 1;
+    const int sl = (ml & 31) ^ (2 * g + hh + 8 * (i & 1));
+    const unsigned char* rp = lds + (((i * NJ + (ml >> 5)) * 4 + g) * 64 + hh * 32 + sl) * 16;
+    f32x4 v = *reinterpret_cast<const f32x4*>(rp);
+#pragma unroll
+    for (int w = 1; w < KS; ++w) v += *reinterpret_cast<const f32x4*>(rp + w * RED);
+    const int m = m0 + ml, nn = n0 + 4 * q;
+    if (m >= M) continue;
+    uint16_t* p = y + int64_t(m) * ldy + nn;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (F4) v[e] *= alpha;
+      if (beta && nn + e < N) v[e] += bf2f(p[e]);
+    }
+    if (vec && nn + 3 < N) {
+      *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (nn + e < N) p[e] = f2bf(v[e]);
+    }
+  }
 }
 
 }  // namespace
@@ -702,15 +939,74 @@ hipError_t launch_mxfp8_quant(const uint16_t* x, int64_t ldx, int64_t rows, int6
   return hipGetLastError();
 }
 
+namespace {
+
+// The tile of a GEMM, by its estimated time in us: f0 + rounds (f + a nst), nst K stages of
+// 128 bytes, rounds of 256 CUs x occ work-groups; `alone` replaces a where two work-groups
+// fit a CU and no more than 256 run. The figures are fits to sweeps of M 1 .. 8192, N and K
+// 1024 .. 12288 on an MI355X, operands rotating through 3 buffers (us, best of the others):
+//   M     N     K       256 x 256  256 x 128  128 x 128  64 x 64   64 x 64   64 x 32  32 x 32
+//                                                        4 waves   2 waves
+//   1     3072  3072    28.2       17.6       11.9       7.2       8.6       6.2      5.0
+//   1     12288 12288   128        80         55         36        36        34       35
+//   33    5120  5120    44         27         18         11.3      12.8      9.5      11.0
+//   256   3072  3072    34         20.6       14.6       9.1       10.2      13.3     11.4
+//   512   3072  3072    34         20.7       14.8       16.5      13.0      19.8     19.8
+//   256   12288 3072    35         21.1       15.6       25.6      24.9      37       37
+//   2048  3072  3072    33         23.1       30         64        44        80       90
+//   3000  3072  3072    35         43         44         92        75        116      129
+// The large tiles move fewer bytes per product and lose where they leave CUs idle; below
+// them the time is the latency of K in series, which the K-split tiles divide by their waves.
+enum GemmKind { kG256, kG256x128, kG128, kGk64, kGk64w2, kGk64x32, kGk32, kGKinds };
+struct GemmTile {
+  int tn, tm, occ;
+  double f0, f, a, alone;
+};
+constexpr GemmTile kMxTiles[kGKinds] = {
+    {256, 256, 1, 2.0, 8.0, 1.05, 0}, {256, 128, 1, 0, 7.0, 0.58, 0},      {128, 128, 1, 0, 5.5, 0.39, 0},
+    {64, 64, 1, 1.5, 3.4, 0.175, 0},  {64, 64, 2, 1.1, 3.9, 0.325, 0.226}, {64, 32, 1, 1.2, 3.0, 0.13, 0},
+    {32, 32, 2, 0.5, 2.8, 0.20, 0.095}};
+GemmKind gemm_plan(const GemmTile (&tiles)[kGKinds], int M, int N, int nst) {
+  int best = 0;
+  double bt = 0;
+  for (int k = 0; k < kGKinds; ++k) {
+    const GemmTile& t = tiles[k];
+    const int64_t n = int64_t((N + t.tn - 1) / t.tn) * ((M + t.tm - 1) / t.tm);
+    const double rounds = double((n + 256 * t.occ - 1) / (256 * t.occ));
+    const double us = t.f0 + rounds * (t.f + nst * (t.occ == 2 && n <= 256 ? t.alone : t.a));
+    if (k == 0 || us < bt) best = k, bt = us;
+  }
+  return GemmKind(best);
+}
+GemmKind mxfp8_plan(int M, int N, int K) { return gemm_plan(kMxTiles, M, N, (K + kStage - 1) / kStage); }
+
+}  // namespace
+
 // Preconditions (checked by the caller): K % 32 == 0, (N + 255) / 256 * 256 * K < 2^31,
 // same for M; beta 0 or 1.
 hipError_t launch_mxfp8_gemm(const uint8_t* wq, const uint8_t* wsf, const uint8_t* xq, const uint8_t* xsf,
                              uint16_t* y, int64_t ldy, int M, int N, int K, int beta, hipStream_t s) {
-  const int ntn = (N + kTile - 1) / kTile, ntm = (M + kTile - 1) / kTile;
+  const GemmKind kind = mxfp8_plan(M, N, K);
+  const int tn = kMxTiles[kind].tn, tm = kMxTiles[kind].tm, ntn = (N + tn - 1) / tn, ntm = (M + tm - 1) / tm;
   const int64_t blocks = int64_t(ntn) * ntm;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((mxfp8_gemm<4, 4>), dim3(unsigned(blocks)), dim3(256), 0, s, wq, wsf, xq, xsf, y, ldy, M, N, K, beta,
-                     ntn, ntm);
+  const dim3 grid{unsigned(blocks)};
+  auto tiles = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, wq, wsf, xq, xsf, y, ldy, M, N, K, beta, ntn, ntm);
+  };
+  auto ksplit = [&](auto kern, int ks) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * ks), 0, s, wq, wsf, (const float*)nullptr, xq, xsf, (const float*)nullptr,
+                       y, ldy, M, N, K, beta, ntm);
+  };
+  switch (kind) {
+    case kG256x128: tiles(mxfp8_gemm<4, 2, 3>); break;
+    case kG128: tiles(mxfp8_gemm<2, 2, 4>); break;
+    case kGk64: ksplit(gemm_ksplit<false, 2, 2, 4, 2>, 4); break;
+    case kGk64w2: ksplit(gemm_ksplit<false, 2, 2, 2, 2>, 2); break;
+    case kGk64x32: ksplit(gemm_ksplit<false, 2, 1, 4, 3>, 4); break;
+    case kGk32: ksplit(gemm_ksplit<false, 1, 1, 4, 2>, 4); break;
+    default: tiles(mxfp8_gemm<4, 4, 2>); break;
+  }
   return hipGetLastError();
 }
 

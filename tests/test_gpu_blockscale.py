@@ -143,6 +143,50 @@ def test_gemm_full_size_sampled_rows(cuda):
     assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) - tol))
 
 
+# One shape per output tile that the GEMM chooses by its size (32 x 32, 64 x 32, 64 x 64 with
+# K split over four and two waves, 128 x 128, 256 x 128, 256 x 256), each with ragged rows and
+# columns and a K that is no whole number of 128-byte stages (nor of turns of the stage
+# ring), padded, odd (element-wise stores) and accumulating outputs among them.
+TILES = [
+    (33, 8130, 160, 1, 0.0), (45, 6010, 1120, 6, 1.0), (40, 9000, 96, 0, 0.0), (40, 5000, 2080, 2, 1.0),
+    (200, 5000, 608, 0, 0.0), (257, 8130, 608, 1, 1.0), (700, 6200, 736, 4, 0.0), (1500, 6100, 352, 3, 1.0),
+]
+
+
+def _sampled_rows_match(mode, M, N, K, pad, beta, cuda):
+    """Output rows around every tile edge against the oracle GEMM of those rows."""
+    print(f"{mode.name} gemm tiles M={M} N={N} K={K} pad={pad} beta={beta}", flush=True)
+    rng = np.random.default_rng(M + 3 * N + K)
+    xb = oracle.f32_to_bf16((rng.standard_normal((M, K)) * 2).astype(np.float32))
+    wb = oracle.f32_to_bf16((rng.standard_normal((N, K)) * 0.05).astype(np.float32))
+    to = lambda a: torch.from_numpy(a.view(np.int16)).to(cuda)
+    quant = _quant if mode == QMode.MXFP8 else _quant4
+    X, W = quant(to(xb), M, K, cuda), quant(to(wb), N, K, cuda)
+    y0 = oracle.f32_to_bf16(rng.standard_normal((M, N + pad)).astype(np.float32))
+    y = to(y0).clone()
+    gemm_blockscaled(mode, QMat(*W), QMat(*X), y, N + pad, M, N, K, beta)
+    torch.cuda.synchronize()
+    got = oracle.bf16_to_f32(y.cpu().numpy().view(np.uint16)).astype(np.float64)
+    rows = np.array(sorted({r for t in (0, 32, 64, 128, 192, 256, M) for r in (t - 1, t) if 0 <= r < M}))
+    if mode == QMode.MXFP8:
+        want = oracle.gemm_mxfp8(*oracle.mxfp8_quantize(wb, N, K), *oracle.mxfp8_quantize(xb[rows], len(rows), K),
+                                 len(rows), N, K)
+    else:
+        xq, xs, xa = oracle.nvfp4_quantize(xb, M, K)  # the tensor's amax is over all rows
+        want = oracle.gemm_nvfp4(*oracle.nvfp4_quantize(wb, N, K), xq[rows], xs[rows], xa, len(rows), N, K)
+    old = oracle.bf16_to_f32(y0).astype(np.float64)
+    want = want.astype(np.float64) + (old[rows, :N] if beta else 0.0)
+    # fp32 accumulation, then one bf16 rounding (plus the bf16 of Y for beta = 1)
+    tol = np.abs(want) * 2.0 ** -7 + np.abs(want).max() * 2.0 ** -14
+    assert np.all(np.abs(got[rows, :N] - want) <= tol), float(np.max(np.abs(got[rows, :N] - want) - tol))
+    np.testing.assert_array_equal(got[:, N:], old[:, N:])  # columns past N untouched
+
+
+@pytest.mark.parametrize("M,N,K,pad,beta", TILES)
+def test_gemm_tile_kinds(cuda, M, N, K, pad, beta):
+    _sampled_rows_match(QMode.MXFP8, M, N, K, pad, beta, cuda)
+
+
 # ---------------- NVFP4 (reference blockscale.cu NVFP4 branch) ----------------
 
 def _quant4(x, rows, K, cuda, ldx=None):
