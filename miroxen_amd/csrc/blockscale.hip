@@ -139,7 +139,7 @@ __device__ __forceinline__ void dma_stage(__amdgpu_buffer_rsrc_t rs, const OpAdd
 
 // Epilogue through LDS: the TN x TM = 64 NI x 64 NJ bf16 Y tile (row m = 128 NI bytes of
 // n) fills the stage buffers. Lane (m = lane % 32 of block j, h = lane / 32) holds n = 8g
-// + 4h + (0..3) of block i; the 16-byte chunks of row m are XOR'd within groups of 8 or 16
+// + 4h + (0..3) of block i; the 16-byte chunks of row m are XOR'd with m % 16
 // so that 16 rows' same chunk covers every bank: the 8-byte writes and the 16-byte row
 // reads are free of bank conflicts, and each row goes out as coalesced 16-byte stores.
 // ALPHA: Y = alpha * C (+ Y).
@@ -148,22 +148,19 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[NI][NJ], unsigned
                                            int64_t ldy, int M, int N, int m0, int n0, int wm, int wn, int lane,
                                            int beta, float alpha) {
   constexpr int CH = 8 * NI, RB = 16 * CH;  // chunks and bytes per row
-  auto swz = [](int m) __attribute__((always_inline)) { return NI % 2 == 0 ? m & 15 : (m >> 1) & 7; };
+  static_assert(NI == 2 || NI == 4, "rows of 256 or 512 bytes");
   const int n = lane & 31, h = lane >> 5;
   block_sync();  // every wave is done with the operand buffers
   {
-    const int xs = swz(n);  // wm and 32 j are multiples of 16
+    const int xs = n & 15;  // m % 16: wm and 32 j are multiples of 16
     unsigned char* wp = lds + (wm + n) * RB + 8 * h + wn * 2;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        // chunk of the row: wn / 8 + 4 i + g. wn is 0 or 32 NI; the XOR stays within the
-        // wave's chunks when 4 NI is a multiple of its span, else it is taken on the whole
+        // chunk wn / 8 + 4 i + g of the row; NI = 4: wn / 8 is 0 or 16, outside the XOR
         const int q = 4 * i + g;
-        unsigned char* wq = (4 * NI) % (NI % 2 == 0 ? 16 : 8) == 0
-                                ? wp + ((q ^ xs) << 4)
-                                : lds + (wm + n) * RB + 8 * h + (((wn >> 3) + q) ^ xs) * 16;
+        unsigned char* wq = NI == 4 ? wp + ((q ^ xs) << 4) : lds + (wm + n) * RB + 8 * h + (((wn >> 3) + q) ^ xs) * 16;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           const f32x16& c = acc[i][j];
@@ -191,7 +188,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[NI][NJ], unsigned
   for (int it = 0; it < 2 * NJ * NI; ++it) {
     const int idx = it * 256 + int(threadIdx.x), r = idx / CH, c = idx % CH, m = m0 + r, nn = n0 + 8 * c;
     if (m >= M) break;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * RB + ((c ^ swz(r)) << 4));
+    const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * RB + ((c ^ (r & 15)) << 4));
     uint16_t* p = y + int64_t(m) * ldy + nn;
     if (vec && nn + 7 < N) {
       *reinterpret_cast<u32x4*>(p) = v;
@@ -207,32 +204,20 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[NI][NJ], unsigned
 // the reference's 128 x 4 interleaved layout: byte (r / 128) kbp 128 + (kb / 4) 512 +
 // (r % 32) 16 + ((r % 128) / 32) 4 + kb % 4. A 128-row band puts its four row blocks next
 // to each other, so aligned runs of 4 or 2 blocks are one 16- or 8-byte load per lane.
-template <int NB>
-struct ScaleAddr {
-  uint32_t off[NB == 3 ? 3 : 1];
-};
-template <int NB>
-__device__ __forceinline__ ScaleAddr<NB> scale_addr(int row0, int kbp, int n) {
-  ScaleAddr<NB> a;
-#pragma unroll
-  for (int b = 0; b < (NB == 3 ? 3 : 1); ++b) {
-    const int r = row0 + 32 * b;
-    a.off[b] = uint32_t(r / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n) + uint32_t((r % 128) / 32) * 4u;
-  }
-  return a;
+__device__ __forceinline__ uint32_t scale_addr(int row0, int kbp, int n) {
+  return uint32_t(row0 / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n) + uint32_t((row0 % 128) / 32) * 4u;
 }
 template <int NB>
-__device__ __forceinline__ void scale_load(__amdgpu_buffer_rsrc_t rs, const ScaleAddr<NB>& a, uint32_t soff,
-                                           uint32_t (&w)[NB]) {
+__device__ __forceinline__ void scale_load(__amdgpu_buffer_rsrc_t rs, uint32_t off, uint32_t soff, uint32_t (&w)[NB]) {
+  static_assert(NB == 1 || NB == 2 || NB == 4, "an aligned run of row blocks");
   if constexpr (NB == 4) {
-    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, a.off[0], soff, 0));
+    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, soff, 0));
     w[0] = v[0], w[1] = v[1], w[2] = v[2], w[3] = v[3];
   } else if constexpr (NB == 2) {
-    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, a.off[0], soff, 0));
+    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, soff, 0));
     w[0] = v[0], w[1] = v[1];
   } else {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) w[b] = __builtin_amdgcn_raw_buffer_load_b32(rs, a.off[b], soff, 0);
+    w[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, off, soff, 0);
   }
 }
 
@@ -294,8 +279,8 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   const int n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rsw = buf_rsrc(wsf, uint32_t(pad_up(N, 128) * kbp));
   const __amdgpu_buffer_rsrc_t rsx = buf_rsrc(xsf, uint32_t(pad_up(M, 128) * kbp));
-  const ScaleAddr<NI> sw = scale_addr<NI>(n0 + wn, kbp, n);
-  const ScaleAddr<NJ> sx = scale_addr<NJ>(m0 + wm, kbp, n);
+  const uint32_t sw = scale_addr(n0 + wn, kbp, n);
+  const uint32_t sx = scale_addr(m0 + wm, kbp, n);
 
   // LDS operand reads: rows row0 + n of an operand tile for K step s. In the f8
   // operand of the 32x32x64 MFMA, bytes 0-15 of lane half h are K 16h .. 16h+15 and
@@ -329,7 +314,7 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   // on stage st's buffer is free and takes stage st + NBUF: its DMA op u goes into slot SL +
   // PRE + 5/8 * 2 SL * u / ND, the last ones into the first slots of stage st + 1.
   constexpr int SL = NI * NJ, PRE = SL >= 8 ? 2 : 1, ND = 2 * (NI + NJ), NP = 2 * (NI + NJ);
-  constexpr int SCL = (NI == 3 ? 3 : 1) + (NJ == 3 ? 3 : 1);  // scale loads per stage
+  constexpr int SCL = 2;  // scale loads per stage
   auto dma_slot = [](int u) constexpr { return SL + PRE + u * 5 * SL / (4 * ND); };
   static_assert(dma_slot(ND - 1) < 3 * SL, "a stage's DMA ends before its wait");
   // DMA op u: operand u & 1 (X's ops run out first or last when NI != NJ), index u >> 1
@@ -586,24 +571,33 @@ __global__ void __launch_bounds__(256) nvfp4_quant(const uint16_t* __restrict__ 
   sf[so] = uint8_t(se);
 }
 
-// NVFP4 GEMM: the MXFP8 kernel's tiling (256 n x 256 m per 4-wave work-group, 128 x 128
-// per wave, 256 fp32 accumulators in AGPRs, K stages of 128 bytes = 256 values DMA'd
-// into LDS with the same swizzle, XCD-grouped tile order, LDS epilogue), but the raw e2m1
+// NVFP4 GEMM: the MXFP8 kernel's tiling (64 NI n x 64 NJ m per 4-wave work-group, fp32
+// accumulators in AGPRs, K stages of 128 bytes = 256 values DMA'd into LDS
+// with the same swizzle, XCD-grouped tile order, LDS epilogue), but the raw e2m1
 // data is dequantized in registers and multiplied on the f16 MFMA (32x32x16). gfx950's
 // scaled MFMA takes one power-of-two scale per 32 values, NVFP4 an e4m3 scale per 16;
-// the product of an e2m1 value and an e4m3 scale has at most 5 significant bits, so
+// the product of an e2m1 value and an e4m3 scale has at most 6 significant bits, so
 // e2m1 -> f16 (v_cvt_scalef32_pk_f16_fp4, scale 1) times the block scale in f16
 // (v_pk_mul_f16) is exact, as are the MFMA's f16 products; accumulation is fp32, and
 // alpha = gW gX scales the tile in the epilogue.
 //
 // Operand layout: the MFMA sums its 16 K values in any order, so the two lane halves
-// take different 16-value blocks: for 32-value chunk c of a stage, lane half h of row
-// r reads the 8 bytes of block 2c + h (one ds_read_b64) and feeds values 0-7 of it to
-// MFMA step 2c and values 8-15 to step 2c + 1; W and X use the same assignment, so
-// every product pairs the same K. One e4m3 scale per lane per chunk and operand block.
+// take different 16-value blocks: lane half h of row r reads the 16 bytes of chunk 2c + h
+// of a stage (blocks 4c + 2h + u, u = 0, 1) and feeds bytes 8u + 4w .. + 3 of them to MFMA
+// step 4c + 2u + w; W and X use the same assignment, so every product pairs the same K.
+//
+// What bounds it: a step is NI NJ MFMAs of 32 cycles and 8 (NI + NJ) vector instructions of
+// dequantization (4 x 4: 16 and 64), which fit beside the MFMAs only if they are spread
+// between them. So the next step's operands are dequantized into a second register set while
+// this step's MFMAs run, half a block after each MFMA, in a fixed order (MXA_SCHED); the
+// compiler's own order put the dequantization of a step before its MFMAs, and 8-byte LDS
+// reads of half a chunk waited for each other. M 4096 N 3072 K 12288: 327 -> 227 us (1.36
+// PFLOP/s); M 8192 N 12288 K 4096: 660 -> 576 us (1.43 PFLOP/s, near the rate at which this
+// chip's power limit holds bf16 library GEMMs: 1.4-1.6).
 using f16x2 = __attribute__((ext_vector_type(2))) _Float16;
 using f16x8 = __attribute__((ext_vector_type(8))) _Float16;
 
+// Eight e2m1 values (a dword) times their block's scale in f16.
 __device__ __forceinline__ f16x8 fp4x8_to_f16(uint32_t d, f16x2 s) {
   const f16x2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.f, 0) * s;
   const f16x2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(d, 1.f, 1) * s;
@@ -612,109 +606,153 @@ __device__ __forceinline__ f16x8 fp4x8_to_f16(uint32_t d, f16x2 s) {
   return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], e[0], e[1]};
 }
 
-// A block scale (the low byte) in f16, both halves of the pair.
-__device__ __forceinline__ f16x2 fp4_scale(uint32_t byte) {
-  const float f = __builtin_amdgcn_cvt_f32_fp8(int(byte), 0);
-  return __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(f, f));
+// The block scales in the low two bytes of a word, as an f16 pair (exact).
+__device__ __forceinline__ f16x2 fp4_scales(uint32_t word) {
+  return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(word, 1.f, false);
 }
+__device__ __forceinline__ f16x2 splat16(f16x2 p, int u) { return u ? p.yy : p.xx; }
 __device__ __forceinline__ float fp4_alpha(float aw, float ax) {
   return (aw > 0.f ? aw / kFp4Range : 1.f) * (ax > 0.f ? ax / kFp4Range : 1.f);
 }
 
+template <int NI, int NJ>
 __global__ void __launch_bounds__(256, 1)
 nvfp4_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, const float* __restrict__ wamax,
            const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xsf, const float* __restrict__ xamax,
            uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K, int beta, int ntn, int ntm) {
-  __shared__ __align__(16) unsigned char lds[4 * kStageB];
-  // stage buffers: operand W at lds + bi * kStageB, operand X at lds + (2 + bi) * kStageB
+  constexpr int TN = 64 * NI, TM = 64 * NJ, SA = TN * kStage, SB = TM * kStage;
+  constexpr int NV = 2 * (NI > NJ ? NI : NJ);
+  // stage buffers: operand W at lds + (st & 1) * SA, operand X at lds + 2 SA + (st & 1) * SB
+  __shared__ __align__(16) unsigned char lds[2 * (SA + SB)];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const int gsz = kGroupM * ntn, grp = L / gsz, fm = grp * kGroupM;
   const int gm = min(ntm - fm, kGroupM), li = L - grp * gsz;
-  const int tm = fm + li % gm, tn = li / gm;
-  const int n0 = tn * kTile, m0 = tm * kTile;
-  const int wn = (wave & 1) * 128, wm = (wave >> 1) * 128;
+  const int n0 = li / gm * TN, m0 = (fm + li % gm) * TM;
+  const int wn = (wave & 1) * (32 * NI), wm = (wave >> 1) * (32 * NJ);
   const int RB = K / 2;                                  // bytes per row
   const int kbp = int(pad_up(K / kFp4Block, 4));
   const int nst = (RB + kStage - 1) / kStage;            // stages of 256 values
 
   const __amdgpu_buffer_rsrc_t rw = buf_rsrc(wq + int64_t(n0) * RB, uint32_t(int64_t(N - n0) * RB));
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xq + int64_t(m0) * RB, uint32_t(int64_t(M - m0) * RB));
-  const OpAddr<8> oa = op_addr<8>(RB, lane, wave_u);
-  // Scales: a wave's 128 rows are one 128-row band; lane n's bytes for row blocks b =
-  // 0..3 (r % 32 = n, (r % 128) / 32 = b) and K blocks 4t..4t+3 are the 16 bytes at
-  // band + t 512 + 16 n (word b, byte kb % 4). A stage's 16 blocks: 4 loads per operand.
+  const OpAddr<NV> oa = op_addr<NV>(RB, lane, wave_u);
   const int n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rsw = buf_rsrc(wsf, uint32_t(pad_up(N, 128) * kbp));
   const __amdgpu_buffer_rsrc_t rsx = buf_rsrc(xsf, uint32_t(pad_up(M, 128) * kbp));
-  const uint32_t sw_off = uint32_t((n0 + wn) / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n);
-  const uint32_t sx_off = uint32_t((m0 + wm) / 128) * uint32_t(kbp) * 128u + uint32_t(16 * n);
-  auto fetch = [&](int st, int bi, u32x4 (&sa)[4], u32x4 (&sb)[4]) __attribute__((always_inline)) {
-    dma_stage(rw, oa, RB, st * kStage, lds + bi * kStageB, wave_u);
-    dma_stage(rx, oa, RB, st * kStage, lds + (2 + bi) * kStageB, wave_u);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      sa[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsw, sw_off + uint32_t((4 * st + t) * 512), 0, 0));
-      sb[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsx, sx_off + uint32_t((4 * st + t) * 512), 0, 0));
-    }
-  };
-  // LDS read address of (row block b, chunk c): row (w* + 32 b + n), logical 16-byte
-  // chunk c at physical c ^ ((row >> 1) & 7), this half's 8 bytes
+  const uint32_t sw = scale_addr(n0 + wn, kbp, n);
+  const uint32_t sx = scale_addr(m0 + wm, kbp, n);
+  // LDS address of this half's chunk 2c + h of row (w* + 32 b + n): physical chunk
+  // (2c + h) ^ ((row >> 1) & 7)
   const int x = (n >> 1) & 7;
-  const int abase = (wn + n) * kStage + 8 * h, bbase = (wm + n) * kStage + 8 * h;
-  // the block scale of (row block b, chunk c) in f16, both halves of the pair
-  auto scale_of = [&](const u32x4 (&sw)[4], int b, int c) __attribute__((always_inline)) -> f16x2 {
-    return fp4_scale(sw[c >> 1][b] >> (8 * (2 * (c & 1) + h)));
-  };
+  int co[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) co[c] = ((2 * c + h) ^ x) << 4;
+  const int abase = (wn + n) * kStage, bbase = 2 * SA + (wm + n) * kStage;
 
-  f32x16 acc[4][4];
+  f32x16 acc[NI][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       acc[i][j] = f32x16{};
       asm volatile("" : "+a"(acc[i][j]));
     }
 
-  u32x4 sa[4], sb[4], na[4], nb[4];
-  fetch(0, 0, na, nb);
+  constexpr int SL = NI * NJ, NB = NI + NJ, ND = 2 * NB;
+  uint32_t wa[4][NI], wb[4][NJ];  // scale words of K blocks 4c .. 4c + 3 of a stage
+  i32x4 raw[2][NB];               // e2m1 chunks of c (by parity): NI W blocks, then NJ X blocks
+  f16x2 ps[2][NB];                // their two block scales
+  f16x8 op[2][NB];                // dequantized operands of a step (by parity)
+  auto words = [&](int st, auto cc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value;
+    const uint32_t so = uint32_t(min(4 * st + c, kbp / 4 - 1) * 512);  // (past the end: never used)
+    scale_load<NI>(rsw, sw, so, wa[c]);
+    scale_load<NJ>(rsx, sx, so, wb[c]);
+  };
+  auto read = [&](int buf, auto cc, auto bc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value, b = decltype(bc)::value;
+    const unsigned char* p = b < NI ? lds + abase + buf * SA + b * 32 * kStage : lds + bbase + buf * SB + (b - NI) * 32 * kStage;
+    raw[c & 1][b] = *reinterpret_cast<const i32x4*>(p + co[c]);
+  };
+  auto scale = [&](auto cc, auto bc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value, b = decltype(bc)::value;
+    ps[c & 1][b] = fp4_scales((b < NI ? wa[c][b < NI ? b : 0] : wb[c][b < NI ? 0 : b - NI]) >> (16 * h));
+  };
+  // dequantization unit d (0 .. 2 NB - 1) of step k: half (4 values) of one block, in the
+  // order the MFMAs need the blocks: W 0, X 0 .. NJ - 1, W 1 ..
+  auto deq = [&](auto kc, auto dc) __attribute__((always_inline)) {
+    constexpr int k = decltype(kc)::value, c = k >> 2, u = (k >> 1) & 1, w = k & 1;
+    constexpr int o = decltype(dc)::value >> 1, hi = decltype(dc)::value & 1;
+    constexpr int b = o == 0 ? 0 : o <= NJ ? NI + o - 1 : o - NJ;
+    const uint32_t v = uint32_t(raw[c & 1][b][2 * u + w]);
+    const f16x2 s = splat16(ps[c & 1][b], u);
+    const f16x2 e = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 1.f, 2 * hi) * s;
+    const f16x2 f = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 1.f, 2 * hi + 1) * s;
+    f16x8& d = op[k & 1][b];
+    d[4 * hi] = e[0], d[4 * hi + 1] = e[1], d[4 * hi + 2] = f[0], d[4 * hi + 3] = f[1];
+  };
+  auto dma = [&](auto uc, int st, uint32_t past) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value, lo = 2 * (NI < NJ ? NI : NJ);
+    constexpr bool isx = u < 2 * lo ? (u & 1) : NJ > NI;
+    constexpr int jj = u < 2 * lo ? u >> 1 : u - lo;
+    if constexpr (isx) dma_op(rx, oa, jj, past, st * kStage, lds + 2 * SA + (st & 1) * SB, wave_u);
+    else dma_op(rw, oa, jj, past, st * kStage, lds + (st & 1) * SA, wave_u);
+  };
+  using C0 = std::integral_constant<int, 0>;
+  // (the words first: the compiler waits for them by the number of younger loads)
+  static_for<4>([&](auto c) __attribute__((always_inline)) { words(0, c); });
+  static_for<ND>([&](auto u) __attribute__((always_inline)) { dma(u, 0, past_k(oa, RB, 0)); });
+  wait_vm();
+  block_sync();
+  static_for<NB>([&](auto b) __attribute__((always_inline)) {
+    read(0, C0{}, b);
+    scale(C0{}, b);
+  });
+  MXA_SCHED;
+  words(1, C0{});
+  static_for<ND>([&](auto u) __attribute__((always_inline)) { dma(u, 1, past_k(oa, RB, kStage)); });
+  static_for<2 * NB>([&](auto d) __attribute__((always_inline)) { deq(C0{}, d); });
+  MXA_SCHED;
+
+  // A stage is 16 steps of SL MFMA slots. Beside step k's MFMAs: step k + 1's dequantization;
+  // in steps 4c + 1 and 4c + 2 the LDS reads and block scales of chunk c + 1; in step 13 the
+  // stage barrier (stage st + 1 landed; every wave holds the last chunk of stage st in
+  // registers), from then on the DMA of stage st + 2; a chunk's scale words of the next stage
+  // as soon as this stage's are consumed.
   for (int st = 0; st < nst; ++st) {
-    const int bi = st & 1;
-    wait_vm();     // this wave's DMA of stage st and its scale words landed ...
-    block_sync();  // ... for every wave, and every wave is done with stage st - 1
-#pragma unroll
-    for (int t = 0; t < 4; ++t) sa[t] = na[t], sb[t] = nb[t];
-    if (st + 1 < nst) fetch(st + 1, bi ^ 1, na, nb);
-    const unsigned char* ca = lds + bi * kStageB;
-    const unsigned char* cb = lds + (2 + bi) * kStageB;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      u32x2 ra[4], rb[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int co = ((c ^ x) << 4) + b * 32 * kStage;
-        ra[b] = *reinterpret_cast<const u32x2*>(ca + abase + co);
-        rb[b] = *reinterpret_cast<const u32x2*>(cb + bbase + co);
+    const int buf = st & 1;
+    const uint32_t past = past_k(oa, RB, (st + 2) * kStage);
+    static_for<16>([&](auto kc) __attribute__((always_inline)) {
+      constexpr int k = decltype(kc)::value, c = k >> 2, r = k & 3, cn = (c + 1) & 3;
+      if constexpr (k == 13) {
+        wait_vm();
+        block_sync();
+        MXA_SCHED;
       }
-      f16x2 psa[4], psb[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) psa[b] = scale_of(sa, b, c), psb[b] = scale_of(sb, b, c);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        f16x8 av[4], bv[4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) av[b] = fp4x8_to_f16(ra[b][u], psa[b]), bv[b] = fp4x8_to_f16(rb[b][u], psb[b]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
-      }
-    }
+      static_for<SL>([&](auto qc) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value, i = q / NJ, j = q % NJ;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(op[k & 1][i], op[k & 1][NI + j], acc[i][j], 0, 0, 0);
+        static_for<2 * NB>([&](auto d) __attribute__((always_inline)) {
+          if constexpr (decltype(d)::value * SL / (2 * NB) == q) deq(std::integral_constant<int, (k + 1) & 15>{}, d);
+        });
+        static_for<NB>([&](auto b) __attribute__((always_inline)) {
+          if constexpr (r == 1 && decltype(b)::value * SL / NB == q)
+            read(c == 3 ? buf ^ 1 : buf, std::integral_constant<int, cn>{}, b);
+          if constexpr (r == 2 && decltype(b)::value * SL / NB == q) scale(std::integral_constant<int, cn>{}, b);
+        });
+        if constexpr (r == 3 && q == 0) words(cn == 0 ? st + 2 : st + 1, std::integral_constant<int, cn>{});
+        if constexpr (k >= 13)
+          static_for<ND>([&](auto u) __attribute__((always_inline)) {
+            if constexpr (decltype(u)::value * 3 * SL / ND == (k - 13) * SL + q) dma(u, st + 2, past);
+          });
+        MXA_SCHED;
+      });
+    });
   }
   wait_vm();  // no LDS-DMA may land after the work-group ends
-  const float alpha = fp4_alpha(*wamax, *xamax);
-  store_tile<4, 4, true>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, alpha);
+  store_tile<NI, NJ, true>(acc, lds, y, ldy, M, N, m0, n0, wm, wn, lane, beta, fp4_alpha(*wamax, *xamax));
 }
 
 // ---------------- GEMM of few tiles: K split over the waves of a work-group ----------------
@@ -756,8 +794,8 @@ gemm_ksplit(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, con
   const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xq + int64_t(m0) * RB, uint32_t(int64_t(M - m0) * RB));
   const __amdgpu_buffer_rsrc_t rsw = buf_rsrc(wsf, uint32_t(pad_up(N, 128) * kbp));
   const __amdgpu_buffer_rsrc_t rsx = buf_rsrc(xsf, uint32_t(pad_up(M, 128) * kbp));
-  const ScaleAddr<NI> sw = scale_addr<NI>(n0, kbp, n);
-  const ScaleAddr<NJ> sx = scale_addr<NJ>(m0, kbp, n);
+  const uint32_t sw = scale_addr(n0, kbp, n);
+  const uint32_t sx = scale_addr(m0, kbp, n);
   // DMA op j (rows 8 j .. 8 j + 7): lane i fills physical chunk i % 8 of row 8 j + i / 8,
   // logical chunk (i % 8) ^ ((row >> 1) & 7), which depends on j through its parity
   constexpr int NV = 4 * (NI > NJ ? NI : NJ);
@@ -854,9 +892,9 @@ gemm_ksplit(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, con
         for (int u = 0; u < 2; ++u) {
           f16x2 pa[NI], pb[NJ];
 #pragma unroll
-          for (int b = 0; b < NI; ++b) pa[b] = fp4_scale(ta[r][b] >> (8 * u));
+          for (int b = 0; b < NI; ++b) pa[b] = splat16(fp4_scales(ta[r][b]), u);
 #pragma unroll
-          for (int b = 0; b < NJ; ++b) pb[b] = fp4_scale(tb[r][b] >> (8 * u));
+          for (int b = 0; b < NJ; ++b) pb[b] = splat16(fp4_scales(tb[r][b]), u);
 #pragma unroll
           for (int w = 0; w < 2; ++w) {
             f16x8 fa[NI], fb[NJ];
@@ -1022,16 +1060,53 @@ hipError_t launch_nvfp4_quant(const uint16_t* x, int64_t ldx, int64_t rows, int6
   return hipGetLastError();
 }
 
+namespace {
+
+// The same estimate for NVFP4 (stages of 256 values; the f16 MFMAs weigh more, so the
+// large tiles hold on to smaller shapes). Measured us, as above:
+//   M     N     K       256 x 256  256 x 128  128 x 128  64 x 64   64 x 64   64 x 32  32 x 32
+//                                                        4 waves   2 waves
+//   1     3072  3072    50         34         22         9.9       14.2      8.2      6.2
+//   1     12288 12288   184        122        84         29        45        22       25
+//   33    5120  5120    81         54         36         14.6      21.7      11.3     13.5
+//   256   3072  3072    54         36         23         11.0      15.6      15.8     12.6
+//   512   3072  3072    55         37         24         20.8      17.5      24       22
+//   1024  3072  3072    55         37         25         31        32        47       40
+//   2048  3072  3072    56         39         43         60        50        90       76
+//   4096  3072  12288   227        283        262        350       337       461      547
+constexpr GemmTile kF4Tiles[kGKinds] = {
+    {256, 256, 1, 0, 8.0, 3.9, 0},   {256, 128, 1, 0, 7.7, 2.4, 0},    {128, 128, 2, 0, 4.4, 3.2, 1.6},
+    {64, 64, 1, 1.0, 4.5, 0.45, 0},  {64, 64, 2, 1.0, 4.2, 1.02, 0.87}, {64, 32, 1, 0.9, 3.7, 0.32, 0},
+    {32, 32, 2, 0.5, 2.7, 0.53, 0.25}};
+GemmKind nvfp4_plan(int M, int N, int K) { return gemm_plan(kF4Tiles, M, N, (K / 2 + kStage - 1) / kStage); }
+
+}  // namespace
+
 // Preconditions (checked by the caller): K % 32 == 0, (N + 255) / 256 * 256 * K / 2 < 2^31,
 // same for M; beta 0 or 1; the amax pointers are device floats written by the quantizer.
 hipError_t launch_nvfp4_gemm(const uint8_t* wq, const uint8_t* wsf, const float* wamax, const uint8_t* xq,
                              const uint8_t* xsf, const float* xamax, uint16_t* y, int64_t ldy, int M, int N, int K,
                              int beta, hipStream_t s) {
-  const int ntn = (N + kTile - 1) / kTile, ntm = (M + kTile - 1) / kTile;
+  const GemmKind kind = nvfp4_plan(M, N, K);
+  const int tn = kF4Tiles[kind].tn, tm = kF4Tiles[kind].tm, ntn = (N + tn - 1) / tn, ntm = (M + tm - 1) / tm;
   const int64_t blocks = int64_t(ntn) * ntm;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(nvfp4_gemm, dim3(unsigned(blocks)), dim3(256), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M,
-                     N, K, beta, ntn, ntm);
+  const dim3 grid{unsigned(blocks)};
+  auto tiles = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntn, ntm);
+  };
+  auto ksplit = [&](auto kern, int ks) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * ks), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntm);
+  };
+  switch (kind) {
+    case kG256x128: tiles(nvfp4_gemm<4, 2>); break;
+    case kG128: tiles(nvfp4_gemm<2, 2>); break;
+    case kGk64: ksplit(gemm_ksplit<true, 2, 2, 4, 2>, 4); break;
+    case kGk64w2: ksplit(gemm_ksplit<true, 2, 2, 2, 2>, 2); break;
+    case kGk64x32: ksplit(gemm_ksplit<true, 2, 1, 4, 3>, 4); break;
+    case kGk32: ksplit(gemm_ksplit<true, 1, 1, 4, 2>, 4); break;
+    default: tiles(nvfp4_gemm<4, 4>); break;
+  }
   return hipGetLastError();
 }
 

@@ -248,6 +248,18 @@ def test_nvfp4_gemm_matches_oracle(cuda, M, N, K, beta):
     np.testing.assert_array_equal(got[:, N:], oracle.bf16_to_f32(y0)[:, N:])
 
 
+# The same choice for NVFP4 (stages of 256 values).
+TILES4 = [
+    (33, 8130, 288, 1, 0.0), (40, 5000, 2080, 2, 1.0), (70, 6000, 1056, 0, 0.0), (300, 4000, 1312, 6, 1.0),
+    (257, 8130, 1120, 1, 1.0), (700, 6200, 1312, 4, 0.0), (1500, 6100, 608, 3, 1.0),
+]
+
+
+@pytest.mark.parametrize("M,N,K,pad,beta", TILES4)
+def test_nvfp4_gemm_tile_kinds(cuda, M, N, K, pad, beta):
+    _sampled_rows_match(QMode.NVFP4, M, N, K, pad, beta, cuda)
+
+
 @pytest.mark.parametrize("M,N,K", [(300, 512, 1024), (129, 384, 4160)])
 def test_nvfp4_reference_cases_and_gates(cuda, M, N, K):
     """The reference's NVFP4 cases and gates (tests/blockscale_test.cpp:93-96, :135-136):
