@@ -198,7 +198,10 @@ def _quant4(x, rows, K, cuda, ldx=None):
     return q, sf, am
 
 
-@pytest.mark.parametrize("rows,K,pad", [(1, 32, 0), (300, 512, 8), (129, 4160, 0), (2048, 3072, 0)])
+@pytest.mark.parametrize("rows,K,pad", [
+    (1, 32, 0), (300, 512, 8), (129, 4160, 0), (2048, 3072, 0),
+    (1, 65536, 0), (16, 4096, 8), (17, 4096, 0), (2048, 32, 8), (2049, 32, 0),  # both sides of the one-launch limit
+])
 def test_nvfp4_quantizer_bit_exact(cuda, rows, K, pad):
     print(f"nvfp4 quant rows={rows} K={K} pad={pad}", flush=True)
     rng = np.random.default_rng(rows * 3 + K)
