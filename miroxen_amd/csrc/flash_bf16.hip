@@ -429,6 +429,23 @@ __device__ __forceinline__ void store_partial(const QBlock<DH>& X, const BfSplit
   sp.ml[blk * 256 + lrow] = f32x4{X.m, X.l, __builtin_ldexpf(1.f, e - 15), 0.f};
 }
 
+// Causal work-group order: the units of one XCD (a run of whole heads when Hq is a multiple of
+// 8) by falling length over all of its heads, so that the long units start first and the
+// short ones fill the end. By head (each head's query tiles in turn) the last head's longest
+// tile starts when half the work is done (32 query heads x 4096: 174 -> 139 us, 24 heads x
+// 4352: 146 -> 123, 64 x 4096: 306 -> 273).
+struct Unit {
+  int head, qtile;
+};
+__device__ __forceinline__ Unit causal_unit(int b, int ntq, int Hq) {
+  if (Hq % 8 == 0) {
+    const int hpx = Hq / 8, x = b % 8, l = b / 8;
+    return {x * hpx + l % hpx, ntq - 1 - l / hpx};
+  }
+  const int L = xcd_remap(b, ntq * Hq);
+  return {L / ntq, ntq - 1 - L % ntq};
+}
+
 // Occupancy: one work-group of 8 waves per CU, two waves per SIMD. The causal kernels
 // state that target (waves_per_eu 2): aiming for three waves per SIMD, the compiler caps
 // a kernel at 168 VGPRs, and the causal tile loop needs 177 (the per-lane diagonal
@@ -463,8 +480,11 @@ flash_bf16_pp(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, co
     su = Lx - part * sp.units;
     L = sp.full + su;
   }
-  // causal: query tiles with the most key tiles first
-  const int head = L / ntq, qtile = CAUSAL ? ntq - 1 - L % ntq : L % ntq;
+  int head = L / ntq, qtile = L % ntq;
+  if constexpr (CAUSAL) {
+    const Unit un = causal_unit(blockIdx.x, ntq, p.Hq);
+    head = un.head, qtile = un.qtile;
+  }
   const int kvh = head / (p.Hq / p.Hkv);
   const int q0 = qtile * QT + wave * 32;
   const int ntk = tiles_needed<CAUSAL>(p, qtile * QT, QT);
