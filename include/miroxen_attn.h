@@ -88,7 +88,8 @@ int mx_flash_attn_uses_mfma(const void* q, const void* k, const void* v, const v
 
 /* No counterpart in the reference (a diagnostic query): how mx_flash_attn splits the
  * work of these parameters on a device with `cus` compute units (cus <= 0: the current
- * device). The first *full units (head, 256-query tile) run whole; each of the last
+ * device). The first *full units (head, 256-query tile) run whole (grids of few units as
+ * 128-query units whose two wave groups share the keys and merge on the CU); each of the last
  * *units units runs as *parts key ranges whose partial outputs a merge kernel combines
  * (parts == 1: no split). A split call keeps its partials in a fixed 16 MiB device
  * region (one per device, calls ordered by an event); only splits whose partials fit it

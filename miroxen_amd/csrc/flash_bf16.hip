@@ -433,7 +433,7 @@ __device__ __forceinline__ void store_partial(const QBlock<DH>& X, const BfSplit
 // 8) by falling length over all of its heads, so that the long units start first and the
 // short ones fill the end. By head (each head's query tiles in turn) the last head's longest
 // tile starts when half the work is done (32 query heads x 4096: 174 -> 139 us, 24 heads x
-// 4352: 146 -> 123, 64 x 4096: 306 -> 273).
+// 4352: 146 -> 123, 64 x 4096: 306 -> 273; 256 units of the KS kernel below: 60 -> 51).
 struct Unit {
   int head, qtile;
 };
@@ -597,6 +597,176 @@ flash_bf16_pp(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, co
 #endif
 }
 
+// ---------------- KS: both wave groups on the same queries, key tiles alternating ----------------
+// The ping-pong kernel above gives each group its own 128 queries, so a work-group holds 256
+// queries and walks all of its key tiles in series. With few units, or causal units of very
+// different length (256 units of 6 to 34 tiles at 2048 queries x 32 heads: the longest one
+// sets the time), that leaves CUs idle. Here a unit is 128 queries: group A (waves 0-3)
+// takes key tiles 0, 2, 4 .., group B (waves 4-7) tiles 1, 3, 5 .. of the same queries, in
+// the same ping-pong periods (in each, one wave of a SIMD issues MFMAs and the other the
+// softmax), and the two partial results are merged through LDS in fp32. Twice the units,
+// half as long each; the price is one more work-group set-up and a merge per 256 queries and
+// twice the K/V tile traffic (each group DMAs its own tiles into its own K and V double
+// buffers: 128 KB).
+//   period 2i+1: A: P V(2i), S(2i+2)      B: softmax(2i+1)
+//   period 2i+2: A: softmax(2i+2)         B: P V(2i+1), S(2i+3)
+// A group waits for its DMA before the barrier that precedes its MFMA period; those ops were
+// issued two periods before. Key tiles at or past nt are skipped by the group (the barriers are
+// not), their loads are clamped to the last tile.
+template <int DH, bool CAUSAL>
+__global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
+flash_bf16_ks(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+              uint16_t* __restrict__ o, mx_attn_params p, float c, uint32_t qsign) {
+  using Dm = Dims<DH>;
+  constexpr int QT = 128, LDK = (Dm::KOPS + 3) / 4, LDV = (Dm::VOPS + 3) / 4;
+  __shared__ __align__(16) unsigned char ka0[Dm::KTB];
+  __shared__ __align__(16) unsigned char ka1[Dm::KTB];
+  __shared__ __align__(16) unsigned char va0[Dm::VTB];
+  __shared__ __align__(16) unsigned char va1[Dm::VTB];
+  __shared__ __align__(16) unsigned char kb0[Dm::KTB];
+  __shared__ __align__(16) unsigned char kb1[Dm::KTB];
+  __shared__ __align__(16) unsigned char vb0[Dm::VTB];
+  __shared__ __align__(16) unsigned char vb1[Dm::VTB];
+  __shared__ uint64_t live_tiles[kMaxLiveTiles];
+  const Lane ln(c);
+  const int wave = threadIdx.x >> 6;
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave), wq = wave_u & 3;
+  const bool group_a = wave_u < 4;
+  const int ntq = (p.Sq + QT - 1) / QT;
+  int head, qtile;
+  if constexpr (CAUSAL) {
+    const Unit u = causal_unit(blockIdx.x, ntq, p.Hq);
+    head = u.head, qtile = u.qtile;
+  } else {
+    const int L = xcd_remap(blockIdx.x, gridDim.x);
+    head = L / ntq, qtile = L % ntq;
+  }
+  const int kvh = head / (p.Hq / p.Hkv);
+  const int q0 = qtile * QT + wq * 32;
+  const int nt = tiles_needed<CAUSAL>(p, qtile * QT, QT);
+  const int64_t kvbase = int64_t(kvh) * DH;
+  const TileAddr ta = tile_addr<4>(p, wq, ln.lane);
+
+  QBlock<DH> A;
+  if (CAUSAL && nt == 0) {  // no visible key for any query of the work-group -> 0
+    if (!group_a) return;
+    qblock_init(A, q, p, q0, head, ln, qsign);
+    store_block(A, o, p, q0, head, ln);
+    return;
+  }
+  const bool mask16 = p.kv_valid && (reinterpret_cast<uintptr_t>(p.kv_valid) & 15) == 0;
+  Live16 lv16{};
+  if (mask16) lv16 = live16_issue<8>(p, nt, wave_u, ln.lane);
+  auto ld_k = [&](int t, unsigned char* d) __attribute__((always_inline)) {
+    load_tile<4, false, DH>(k, t < nt ? t : nt - 1, d, p, kvbase, wq, ta);
+  };
+  auto ld_v = [&](int t, unsigned char* d) __attribute__((always_inline)) {
+    load_tile<4, true, DH>(v, t < nt ? t : nt - 1, d, p, kvbase, wq, ta);
+  };
+  if (group_a) {
+    ld_k(0, ka0), ld_v(0, va0), ld_k(2, ka1);
+  } else {
+    ld_k(1, kb0), ld_v(1, vb0), ld_k(3, kb1);
+  }
+  qblock_init(A, q, p, q0, head, ln, qsign);
+  if (mask16) live16_finish<8>(live_tiles, lv16, p, nt, wave_u, ln.lane);
+  else build_live<8, KT>(live_tiles, p, nt, wave, ln.lane);
+
+  // MFMA period of tile t: P V(t), S(t + 2), and the DMA of V(t + 2) and K(t + 4)
+  auto mfma_part = [&](int t, const unsigned char* kc, const unsigned char* vc, unsigned char* kfree,
+                       unsigned char* vfree) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_setprio(1);
+    ld_v(t + 2, vfree);
+    pv(vc, A, ln);
+    sched_v<4 * Dm::NB, LDV>();
+    ld_k(t + 4, kfree);
+    scores(kc, A, ln);
+    sched_k<2 * Dm::NC, LDK>();
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto valu_part = [&](int t) __attribute__((always_inline)) {
+    const uint64_t live = tile_live<KT>(live_tiles, p, t);
+    const bool diag = CAUSAL && int64_t(p.q_offset) + q0 - int64_t(t) * KT < KT - 1;  // wave-uniform
+    if (live != ~0ull || diag) mask_scores<CAUSAL>(A, live, diag ? causal_rel(p, q0 + ln.n, t) : KT - 1, ln);
+    softmax(A, ln);
+    rescale(A);
+  };
+
+  wait_vm_n<0>();
+  __syncthreads();  // the first tiles and the liveness bitmaps are visible
+  if (group_a) {
+    scores(ka0, A, ln);
+    sched_k<2 * Dm::NC, 0>();
+    block_sync();
+    valu_part(0);
+    auto step = [&](int t, const unsigned char* kc, const unsigned char* vc, unsigned char* kfree,
+                    unsigned char* vfree) __attribute__((always_inline)) {
+      wait_vm_n<0>();
+      block_sync();
+      mfma_part(t, kc, vc, kfree, vfree);
+      block_sync();
+      if (t + 2 < nt) valu_part(t + 2);
+    };
+    for (int t = 0; t < nt; t += 4) {
+      step(t, ka1, va0, ka0, va1);
+      if (t + 2 < nt) step(t + 2, ka0, va1, ka1, va0);
+    }
+  } else {
+    block_sync();
+    scores(kb0, A, ln);
+    sched_k<2 * Dm::NC, 0>();
+    auto step = [&](int t, const unsigned char* kc, const unsigned char* vc, unsigned char* kfree,
+                    unsigned char* vfree) __attribute__((always_inline)) {
+      block_sync();
+      if (t < nt) valu_part(t);
+      wait_vm_n<0>();
+      block_sync();
+      if (t < nt) mfma_part(t, kc, vc, kfree, vfree);
+    };
+    for (int t = 1; t - 1 < nt; t += 4) {
+      step(t, kb1, vb0, kb0, vb1);
+      if (t + 1 < nt) step(t + 2, kb0, vb1, kb1, vb0);
+    }
+  }
+  wait_vm_n<0>();  // no LDS-DMA may land in what follows
+  __syncthreads();
+
+  // Merge: group B's (acc, m, l) through LDS into the group A wave with the same queries.
+  unsigned char* buf = wq == 0 ? va0 : wq == 1 ? va1 : wq == 2 ? vb0 : vb1;  // NB * 4 KB each
+  f32x2* ml = reinterpret_cast<f32x2*>(ka0) + wq * 64 + ln.lane;
+  if (!group_a) {
+#pragma unroll
+    for (int db = 0; db < A.NB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(buf + ((db * 4 + g) * 64 + ln.lane) * 16) =
+            f32x4{A.acc[db][4 * g], A.acc[db][4 * g + 1], A.acc[db][4 * g + 2], A.acc[db][4 * g + 3]};
+    *ml = f32x2{A.m, A.l};
+  }
+  __syncthreads();
+  if (!group_a) return;
+  const f32x2 b = *ml;
+  const float M = fmaxf(A.m, b[0]);
+  const float ca = A.m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(A.m - M);
+  const float cb = b[0] == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(b[0] - M);
+  A.l = A.l * ca + b[1] * cb;
+#pragma unroll
+  for (int db = 0; db < A.NB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(buf + ((db * 4 + g) * 64 + ln.lane) * 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) A.acc[db][4 * g + e] = A.acc[db][4 * g + e] * ca + x[e] * cb;
+    }
+  if constexpr (DH % 32 == 0) {
+    if ((reinterpret_cast<uintptr_t>(o) & 15) == 0 && (p.o_stride & 7) == 0) {
+      store_block_lds(A, o, p, q0, head, ln, buf);  // (this wave alone reads and writes buf)
+      return;
+    }
+  }
+  store_block(A, o, p, q0, head, ln);
+}
+
 // Merge of the split units' parts: one thread per (query, 8 channels). With
 // M = max m_i and c_i = l_i 2^(m_i - M), o = sum c_i scale_i o_i / sum c_i (parts
 // whose keys were all dead have l_i = 0 and drop out; no live key at all gives 0).
@@ -662,6 +832,25 @@ size_t bf16_split_bytes(int units, int parts, int D) {
 constexpr size_t kBfSplitBytes = size_t(16) << 20;
 static __device__ __align__(256) unsigned char bf16_split_scratch[kBfSplitBytes];
 
+// Whether an unsplit call runs flash_bf16_ks (128-query units, key tiles alternating between
+// the wave groups) instead of flash_bf16_pp (256-query units). Causal: when the 256-query units
+// are one round or less, i.e. when the longest one sets the time (us, pp / ks; 32 query heads:
+// 333 keys 14.6 / 12.4, 1000 34 / 23, 2048 queries x 2165 keys 60.6 / 50.7, 12 heads x 3000
+// 68 / 47; beyond one round pp, 32 x 3000 86 / 94, 32 x 8192 504 / 555). Otherwise by the
+// estimates R (7 + 1.68 ceil(nt / 2)) and R' (6.5 + 1.37 nt) us in R and R' rounds of units,
+// the latter less 15 % where its last round is part of several (fewer busy CUs run at a higher
+// clock): 24 heads x 1088 28.7 / 21.5, x 2600 107 / 87, 16 heads of 72 x 2000 44 / 29, and pp
+// for 24 x 1500 39 / 51, x 2048 53 / 63, x 4352 220 / 255.
+bool use_ks(const mx_attn_params& p, int C) {
+  const int nt = (p.Skv + KT - 1) / KT;
+  const int64_t U = int64_t((p.Sq + 255) / 256) * p.Hq, Uk = int64_t((p.Sq + 127) / 128) * p.Hq;
+  if (C <= 0 || Uk > 0x7fffffff) return false;
+  if (p.causal) return U <= C && nt >= 3;
+  const double rounds = double((U + C - 1) / C), ks_rounds = double((Uk + C - 1) / C);
+  const double pp = rounds * (6.5 + 1.37 * nt) * (rounds > 1 ? 0.85 : 1.0);
+  return ks_rounds * (7.0 + 1.68 * ((nt + 1) / 2)) < 0.97 * pp;
+}
+
 // Split plan for a non-causal grid of U units on C CUs (one work-group per CU). The
 // chip is power-limited: a CU runs a 64-key tile in ~1.29 us (D = 128) while at most
 // ~165 CUs are busy, and the clock drops as more are (~2.0 us per tile with all 256
@@ -681,7 +870,7 @@ Bf16Plan bf16_plan(const mx_attn_params& p, int C) {
   Bf16Plan pl{int(U64), 0, 1};
   if (p.causal || C <= 0 || U64 >= 0x7fffffff) return pl;
   const int U = int(U64), r = U % C;
-  if (r == 0) return pl;
+  if (r == 0 || (U > C && use_ks(p, C))) return pl;
   const double t0 = 1.29e-6 * (0.4 + 0.6 * p.D / 128.0);  // s per tile per CU, <= kBusyFast busy CUs
   constexpr double kBusyFast = 165.0;
   auto tile_s = [&](int busy) { return t0 * (busy > kBusyFast ? busy / kBusyFast : 1.0); };
@@ -759,13 +948,16 @@ hipError_t launch_flash_bf16(const uint16_t* q, const uint16_t* k, const uint16_
 
   Bf16Plan pl{int(blocks), 0, 1};
   SplitDevice* R = nullptr;
-  if (!cz) {
+  bool ks = false;
+  {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < kMaxDev) {
       R = &g_split[dev];
-      pl = bf16_plan(p, device_cus(*R, dev));
+      const int cus = device_cus(*R, dev);
+      pl = bf16_plan(p, cus);  // (causal calls never split)
+      ks = pl.parts == 1 && use_ks(p, cus);
     }
     if (pl.parts > 1) {
       // a captured graph may replay while eager calls use the region: capture runs unsplit
@@ -782,6 +974,12 @@ hipError_t launch_flash_bf16(const uint16_t* q, const uint16_t* k, const uint16_
   };
   auto go = [&](auto DHc) -> hipError_t {
     constexpr int DH = decltype(DHc)::value;
+    if (ks) {
+      const dim3 grid(unsigned((p.Sq + 127) / 128) * unsigned(p.Hq));
+      auto kern = cz ? flash_bf16_ks<DH, true> : flash_bf16_ks<DH, false>;
+      hipLaunchKernelGGL(kern, grid, dim3(512), 0, s, q, k, v, o, p, c, qsign);
+      return hipGetLastError();
+    }
     if (cz) {
       run(flash_bf16_pp<DH, true, false>, blocks);
       return hipGetLastError();

@@ -329,6 +329,47 @@ def test_d72_last_head_ends_the_allocation(cuda):
     assert reference_gate(_f32(out[rows]), want)[0]
 
 
+# Grids of few units run 128-query units whose two wave groups take alternating key tiles and
+# merge in LDS: numbers of key tiles odd and even, the last tile ragged, one group's keys
+# all masked, rows that see no key, ragged query tiles, every head dim, padded and odd output
+# strides (element-wise stores); and causal grids beyond one round of 256-query units, whose
+# order over an XCD's heads differs for head counts that are no multiple of 8.
+# Sq, Skv, Hq, Hkv, D, causal, q_offset, pad, dead keys [lo, hi)
+KS = [
+    (333, 333, 32, 8, 128, 1, 0, 0, (0, 0)), (129, 193, 24, 24, 128, 0, 0, 0, (0, 0)),
+    (1, 257, 40, 8, 128, 1, 256, 0, (0, 0)), (300, 450, 16, 4, 128, 1, -70, 5, (0, 0)),
+    (260, 320, 24, 24, 128, 0, 0, 0, (64, 128)), (200, 250, 24, 24, 128, 0, 0, 3, (128, 250)),
+    (700, 1000, 16, 16, 72, 0, 0, 8, (0, 64)), (513, 300, 16, 8, 72, 1, 40, 6, (0, 0)),
+    (385, 640, 24, 12, 64, 0, 0, 5, (0, 0)), (900, 1000, 8, 8, 64, 1, 100, 0, (300, 400)),
+    (700, 700, 12, 12, 128, 1, 0, 0, (0, 0)),
+    (2100, 2100, 32, 8, 128, 1, 0, 0, (0, 0)), (5600, 5600, 12, 4, 128, 1, 0, 0, (0, 0)),
+]
+
+
+@pytest.mark.parametrize("case", KS, ids=lambda c: "x".join(map(str, c[:5])) + f"_c{c[5]}o{c[6]}p{c[7]}")
+def test_alternating_key_tiles(cuda, case):
+    Sq, Skv, Hq, Hkv, D, causal, off, pad, dead = case
+    print(f"alternating key tiles {case}", flush=True)
+    q, k, v, qs, ks, os_ = _make(Sq, Skv, Hq, Hkv, D, pad, 1.5, 17 + Sq + D, cuda)
+    mask = None
+    if dead[1]:
+        mask = torch.ones(Skv, dtype=torch.uint8)
+        mask[dead[0]:dead[1]] = 0
+    p = AttnParams(Sq=Sq, Skv=Skv, Hq=Hq, Hkv=Hkv, D=D, causal=causal, q_offset=off, q_stride=qs, kv_stride=ks,
+                   o_stride=os_, kv_valid=None if mask is None else mask.to(cuda))
+    out, buf = _run(flash_attn, q, k, v, p, Sq, os_)
+    rows = sorted(set(query_rows(Sq, Hq)) | set(range(0, Sq, max(1, Sq // 29))) | {Sq - 1})
+    got = _f32(out[rows, : Hq * D])
+    want = oracle.attention_f64(_bits(q), _bits(k), _bits(v), Sq, Skv, Hq, Hkv, D, 0.0, causal, off, q_stride=qs,
+                                kv_stride=ks, kv_valid=None if mask is None else mask.numpy(),
+                                rows=np.array(rows, np.int32)).reshape(len(rows), -1)
+    ok, err, tol, rr = reference_gate(got, want)
+    assert ok, f"max_abs={err} limit={tol} rel_rms={rr}"
+    blind = [i for i, r in enumerate(rows) if causal and off + r < 0]
+    assert np.all(got[blind] == 0)
+    _check_guards(buf, 16, Sq, os_, Hq * D, rows)
+
+
 # Key-range split of the grid's last round (flash_attn_split_plan): the split units'
 # rows against the oracle, parts whose keys are all masked, GQA / D = 64 / 72 with
 # padded strides, and repeat / cross-stream calls sharing the library's split region.
