@@ -223,4 +223,14 @@ __device__ __forceinline__ void nr128_row(float (&x)[8], int64_t s, bool valid, 
   for (int r = 0; r < 8; ++r) x[r] = bf2f(f2bf(x[r]));
 }
 
+// nr128_row on 8 packed bf16 channels.
+template <int MODE>
+__device__ __forceinline__ void nr128_words(u32x4& w, int64_t s, bool valid, const NormRope& nr, int lane) {
+  float x[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = bf2f(uint16_t(w[j >> 1] >> ((j & 1) * 16)));
+  nr128_row<MODE>(x, s, valid, nr, lane);
+  w = pack8_bf16(x);
+}
+
 }  // namespace mxa

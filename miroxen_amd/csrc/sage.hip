@@ -25,7 +25,7 @@ namespace {
 
 // ---------------- prologue ----------------
 //
-// Eager calls with Skv <= 8192 (plain prologue) run prep_kv_fused, one launch over K
+// Eager calls with Skv <= 8192 run prep_kv_fused, one launch over K
 // and V (below), plus prep_stats_q's Q blocks when Q is quantized here. Otherwise
 // three launches (the reference uses a memset and four kernels, :433-446):
 //  1. prep_stats_q: blocks [0, Hkv*nb) reduce K/V statistics of one 256-token
@@ -91,75 +91,41 @@ __global__ void __launch_bounds__(256) prep_stats_q(const uint16_t* __restrict__
         for (int r = 0; r < rows; ++r) am = fmaxf(am, fabsf(bf2f(vt_[r * D + d])));
       }
     };
-    if constexpr (NRM < 0) {
-      // every load of a chunk in flight before the first LDS store, and the next chunk's
-      // loads in flight while this one is folded (rows past a chunk's end are not
-      // loaded; their LDS rows are never read)
-      constexpr int NL = kStatChunk * (D / 8) / 256;
-      u32x4 kr[NL], vr[NL];
-      auto load = [&](int64_t c0, int rows) __attribute__((always_inline)) {
+    // every load of a chunk in flight before the first LDS store, and the next chunk's
+    // loads in flight while this one is folded (rows past a chunk's end are not
+    // loaded; their LDS rows are never read)
+    constexpr int NL = kStatChunk * (D / 8) / 256;
+    u32x4 kr[NL], vr[NL];
+    auto load = [&](int64_t c0, int rows) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < NL; ++u) {
-          const int i = tid + 256 * u, r = i / (D / 8), c = (i % (D / 8)) * 8;
-          const int64_t g = (c0 + r) * p.kv_stride + int64_t(h) * D + c;
-          kr[u] = vr[u] = u32x4{0, 0, 0, 0};
-          if (r < rows) {
-            kr[u] = *reinterpret_cast<const u32x4*>(k + g);
-            vr[u] = *reinterpret_cast<const u32x4*>(v + g);
-          }
+      for (int u = 0; u < NL; ++u) {
+        const int i = tid + 256 * u, r = i / (D / 8), c = (i % (D / 8)) * 8;
+        const int64_t g = (c0 + r) * p.kv_stride + int64_t(h) * D + c;
+        kr[u] = vr[u] = u32x4{0, 0, 0, 0};
+        if (r < rows) {
+          kr[u] = *reinterpret_cast<const u32x4*>(k + g);
+          vr[u] = *reinterpret_cast<const u32x4*>(v + g);
         }
-      };
-      const int nch = int((t1 - t0 + kStatChunk - 1) / kStatChunk);  // 1 or 2
-      load(t0, int(t1 - t0 < kStatChunk ? t1 - t0 : kStatChunk));
-      for (int ch = 0; ch < nch; ++ch) {
-        const int64_t c0 = t0 + int64_t(ch) * kStatChunk;
-        const int rows = int(t1 - c0 < kStatChunk ? t1 - c0 : kStatChunk);
-#pragma unroll
-        for (int u = 0; u < NL; ++u) {
-          const int i = tid + 256 * u, r = i / (D / 8), c = (i % (D / 8)) * 8;
-          *reinterpret_cast<u32x4*>(&kt[r * D + c]) = kr[u];
-          *reinterpret_cast<u32x4*>(&vt_[r * D + c]) = vr[u];
-        }
-        __syncthreads();
-        if (ch + 1 < nch) load(c0 + kStatChunk, int(t1 - c0 - kStatChunk < kStatChunk ? t1 - c0 - kStatChunk
-                                                                                       : kStatChunk));
-        fold(rows);
-        __syncthreads();
       }
-    } else {
-      for (int64_t c0 = t0; c0 < t1; c0 += kStatChunk) {
-        const int rows = int(t1 - c0 < kStatChunk ? t1 - c0 : kStatChunk);
-        {
-          // K rows normalised on the way into LDS: one row per 16 lanes, 16 per pass
-          // (all eight rows of a lane group loaded before any is normalised)
-          const int lane = tid & 63, c = (lane & 15) * 8;
-          constexpr int RPG = kStatChunk / 16;  // rows per 16-lane group
-          u32x4 raw[RPG];
+    };
+    const int nch = int((t1 - t0 + kStatChunk - 1) / kStatChunk);  // 1 or 2
+    load(t0, int(t1 - t0 < kStatChunk ? t1 - t0 : kStatChunk));
+    for (int ch = 0; ch < nch; ++ch) {
+      const int64_t c0 = t0 + int64_t(ch) * kStatChunk;
+      const int rows = int(t1 - c0 < kStatChunk ? t1 - c0 : kStatChunk);
 #pragma unroll
-          for (int u = 0; u < RPG; ++u) {
-            const int r = u * 16 + (tid >> 4);
-            raw[u] = u32x4{0, 0, 0, 0};
-            if (r < rows) raw[u] = *reinterpret_cast<const u32x4*>(k + (c0 + r) * p.kv_stride + int64_t(h) * D + c);
-          }
-#pragma unroll
-          for (int u = 0; u < RPG; ++u) {
-            const int r = u * 16 + (tid >> 4);
-            float x[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) x[j] = bf2f(uint16_t(raw[u][j >> 1] >> ((j & 1) * 16)));
-            nr128_row<NRM>(x, c0 + r, r < rows, nk, lane);
-            if (r < rows) *reinterpret_cast<u32x4*>(&kt[r * D + c]) = pack8_bf16(x);
-          }
-          for (int i = tid; i < rows * (D / 8); i += 256) {
-            const int r = i / (D / 8), cc = (i % (D / 8)) * 8;
-            *reinterpret_cast<u32x4*>(&vt_[r * D + cc]) =
-                *reinterpret_cast<const u32x4*>(v + (c0 + r) * p.kv_stride + int64_t(h) * D + cc);
-          }
-        }
-        __syncthreads();
-        fold(rows);
-        __syncthreads();
+      for (int u = 0; u < NL; ++u) {
+        const int i = tid + 256 * u, r = i / (D / 8), c = (i % (D / 8)) * 8;
+        // a row on 16 lanes: K rows are normalised on the way into LDS
+        if constexpr (NRM >= 0) nr128_words<NRM>(kr[u], c0 + r, r < rows, nk, tid & 63);
+        *reinterpret_cast<u32x4*>(&kt[r * D + c]) = kr[u];
+        *reinterpret_cast<u32x4*>(&vt_[r * D + c]) = vr[u];
       }
+      __syncthreads();
+      if (ch + 1 < nch) load(c0 + kStatChunk, int(t1 - c0 - kStatChunk < kStatChunk ? t1 - c0 - kStatChunk
+                                                                                     : kStatChunk));
+      fold(rows);
+      __syncthreads();
     }
     if (tid < D) part[(int64_t(h) * nb + b) * D + tid] = sum / float(p.Skv);
     else if (tid < 2 * D) part[int64_t(p.Hkv) * nb * D + (int64_t(h) * nb + b) * D + (tid - D)] = am;
@@ -438,9 +404,9 @@ __device__ __forceinline__ bool wait_flags(const uint64_t* f, int n, uint64_t ep
 // fallback of a wait that timed out), staged through `sm` in 128-token chunks exactly
 // as prep_stats_q does, stored with device-scope stores. Threads < D: K sum, D..2D-1:
 // V abs-max.
-template <int D>
+template <int D, int NRM>
 __device__ void fused_stats_from_memory(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-                                        const mx_attn_params& p, int h, int b, int nb, float* part,
+                                        const mx_attn_params& p, const NormRope& nk, int h, int b, int nb, float* part,
                                         unsigned char* sm) {
   uint16_t* kt = reinterpret_cast<uint16_t*>(sm);
   uint16_t* vt_ = kt + kStatChunk * D;
@@ -454,7 +420,9 @@ __device__ void fused_stats_from_memory(const uint16_t* __restrict__ k, const ui
     for (int i = tid; i < rows * (D / 8); i += blockDim.x) {
       const int r = i / (D / 8), c = (i % (D / 8)) * 8;
       const int64_t g = (c0 + r) * p.kv_stride + int64_t(h) * D + c;
-      *reinterpret_cast<u32x4*>(&kt[r * D + c]) = *reinterpret_cast<const u32x4*>(k + g);
+      u32x4 kw = *reinterpret_cast<const u32x4*>(k + g);
+      if constexpr (NRM >= 0) nr128_words<NRM>(kw, c0 + r, true, nk, tid & 63);  // (whole 16-lane rows)
+      *reinterpret_cast<u32x4*>(&kt[r * D + c]) = kw;
       *reinterpret_cast<u32x4*>(&vt_[r * D + c]) = *reinterpret_cast<const u32x4*>(v + g);
     }
     __syncthreads();
@@ -472,9 +440,9 @@ __device__ void fused_stats_from_memory(const uint16_t* __restrict__ k, const ui
 // Wait for every block flag of head h (bounded), compute the partials still missing,
 // and return this thread's channel of K mean / V abs-max (threads < D) summed in
 // ascending block order (finalize_channel's arithmetic on device-scope loads).
-template <int D>
+template <int D, int NRM>
 __device__ void fused_fold(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const mx_attn_params& p,
-                           int h, int nb, float* part, const uint64_t* flg, uint64_t epoch, uint64_t ticks,
+                           const NormRope& nk, int h, int nb, float* part, const uint64_t* flg, uint64_t epoch, uint64_t ticks,
                            unsigned char* sm, bool* miss, float& s, float& am) {
   const uint64_t* fh = flg + int64_t(h) * nb;
   if (!wait_flags(fh, nb, epoch, ticks)) {
@@ -482,7 +450,7 @@ __device__ void fused_fold(const uint16_t* __restrict__ k, const uint16_t* __res
       miss[j] = __hip_atomic_load(const_cast<uint64_t*>(fh + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch;
     __syncthreads();
     for (int j = 0; j < nb; ++j)
-      if (miss[j]) fused_stats_from_memory<D>(k, v, p, h, j, nb, part, sm);
+      if (miss[j]) fused_stats_from_memory<D, NRM>(k, v, p, nk, h, j, nb, part, sm);
     wait_vm();
     __syncthreads();
   }
@@ -523,15 +491,18 @@ __device__ void fused_fold(const uint16_t* __restrict__ k, const uint16_t* __res
 
 // One work-group of 512 threads per (head, 256-token block): thread t owns channel
 // chunk c = t % (D/8) (8 channels) of the RPT consecutive tokens from (t / (D/8)) RPT.
-template <int D>
+// NRM >= 0: K rows get norm and RoPE (nk) in registers before anything else is done with them.
+template <int D, int NRM>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) prep_kv_fused(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                      mx_attn_params p, int nb, int64_t skv_pad,
                                                      float* __restrict__ part, float* __restrict__ km,
                                                      float* __restrict__ va, int8_t* __restrict__ ki,
                                                      float* __restrict__ ks, uint8_t* __restrict__ vt,
                                                      u32x4* __restrict__ tab, int* __restrict__ cnt, int ncnt,
-                                                     uint64_t* __restrict__ flg, uint64_t epoch, uint64_t wait_ticks) {
+                                                     uint64_t* __restrict__ flg, uint64_t epoch, uint64_t wait_ticks,
+                                                     NormRope nk) {
   static_assert(D == 64 || D == 128, "head dimension 64 or 128");
+  static_assert(NRM < 0 || D == 128, "the fused norm/rope prologue is built for D = 128");
   constexpr int NT = 512, CPR = D / 8, RPT = kStatTok * CPR / NT;  // chunks per row, tokens per thread
   constexpr int TPT = kKvPad / RPT * CPR;                           // threads per 64-key tile (128)
   static_assert(TPT == 128, "layout");
@@ -564,6 +535,14 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   }
   if (blockIdx.x == 0)  // arrival counters of the attention kernel's split units start at zero
     for (int i = tid; i < ncnt; i += NT) cnt[i] = 0;
+  if constexpr (NRM >= 0) {
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {  // (rows past Skv stay zeros)
+      nr128_words<NRM>(kr[i], t0 + r0 + i, r0 + i < rows, nk, lane);
+      if (r0 + i >= rows) kr[i] = u32x4{0, 0, 0, 0};
+      if (i & 1) __builtin_amdgcn_sched_barrier(0);  // two rows at a time: all eight at once spill
+    }
+  }
 
   // ---- statistics partial: K rows through LDS for the sequential per-channel sum,
   // V abs-max from registers (a max does not depend on order) ----
@@ -638,7 +617,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
 
   // ---- K mean and V abs-max of the head: every work-group folds the partials ----
   float s = 0.f, am = 0.f;
-  fused_fold<D>(k, v, p, h, nb, part, flg, epoch, wait_ticks, sm, miss, s, am);
+  fused_fold<D, NRM>(k, v, p, nk, h, nb, part, flg, epoch, wait_ticks, sm, miss, s, am);
   if (b == 0 && tid < D) {
     km[h * D + tid] = s;
     va[h * D + tid] = am;
@@ -1630,34 +1609,38 @@ hipError_t sage_quantize_d(const uint16_t* q, const uint16_t* k, const uint16_t*
   static_assert(kSqPad % 64 == 0, "Q padding must cover whole 64-row blocks");
   decltype(&prep_stats_q<D, -1, 16>) stats;
   decltype(&prep_kv_quant<D, -1>) kvq;
+  decltype(&prep_kv_fused<D, -1>) fused;
   if constexpr (D == 128) {
     stats = q_group == 64 ? prep_stats_q<D, -1, 64>
           : mode < 0 ? prep_stats_q<D, -1, 16> : mode == kRopeNone ? prep_stats_q<D, kRopeNone, 16>
           : mode == kRopeInterleaved ? prep_stats_q<D, kRopeInterleaved, 16> : prep_stats_q<D, kRopeHalf, 16>;
     kvq = mode < 0 ? prep_kv_quant<D, -1> : mode == kRopeNone ? prep_kv_quant<D, kRopeNone>
         : mode == kRopeInterleaved ? prep_kv_quant<D, kRopeInterleaved> : prep_kv_quant<D, kRopeHalf>;
+    fused = mode < 0 ? prep_kv_fused<D, -1> : mode == kRopeNone ? prep_kv_fused<D, kRopeNone>
+          : mode == kRopeInterleaved ? prep_kv_fused<D, kRopeInterleaved> : prep_kv_fused<D, kRopeHalf>;
   } else {
     if (mode >= 0) return hipErrorInvalidValue;  // the fused norm/rope prologue is D = 128 only
     stats = q_group == 64 ? prep_stats_q<D, -1, 64> : prep_stats_q<D, -1, 16>;
     kvq = prep_kv_quant<D, -1>;
+    fused = prep_kv_fused<D, -1>;
   }
-  // one-pass K/V prologue (prep_kv_fused) for the plain prologue outside stream capture
+  // one-pass K/V prologue (prep_kv_fused) outside stream capture
 #ifdef MX_STAMPS
   const bool debug_old = std::getenv("MX_DEBUG_OLD_PROLOGUE") != nullptr;  // debug builds: A/B of the two paths
 #else
   constexpr bool debug_old = false;
 #endif
-  if (mode < 0 && nb <= kFoldNb && !debug_old) {
+  if (nb <= kFoldNb && !debug_old) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     const hipError_t ce = hipStreamIsCapturing(s, &cap);
     if (ce != hipSuccess) return ce;
     if (cap == hipStreamCaptureStatusNone) {
-      hipLaunchKernelGGL(prep_kv_fused<D>, dim3(unsigned(int64_t(p.Hkv) * nb)), dim3(512), 0, s, k, v, p, nb,
+      hipLaunchKernelGGL(fused, dim3(unsigned(int64_t(p.Hkv) * nb)), dim3(512), 0, s, k, v, p, nb,
                          L.skv_pad, part, km, va, reinterpret_cast<int8_t*>(ws + L.ki),
                          reinterpret_cast<float*>(ws + L.ks), reinterpret_cast<uint8_t*>(ws + L.vt),
                          reinterpret_cast<u32x4*>(ws + L.tab), reinterpret_cast<int*>(ws + L.cnt), L.split_units,
                          reinterpret_cast<uint64_t*>(ws + L.flg), next_epoch(),
-                         g_fused_wait_ticks.load(std::memory_order_relaxed));
+                         g_fused_wait_ticks.load(std::memory_order_relaxed), nk);
       if (!skip_q && qgroups > 0)  // Q blocks only (no statistics blocks: nb = 0)
         hipLaunchKernelGGL(stats, dim3(unsigned((qgroups + 3) / 4)), dim3(256), 0, s, q, k, v, p, 0, qmult,
                            L.sq_pad, part, reinterpret_cast<int8_t*>(ws + L.qi), reinterpret_cast<float*>(ws + L.qs),

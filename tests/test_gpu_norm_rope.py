@@ -127,3 +127,66 @@ def test_fused_norm_rope_prologue_is_bit_exact(cuda, case):
         b = ws2[L2[name]: L2[name] + nb].cpu().numpy()
         assert np.array_equal(a, b), name
     assert torch.equal(o1.view(torch.int16), o2.view(torch.int16))
+
+
+# The one-pass K/V prologue (up to 8192 keys) with norm and RoPE against its separate steps:
+# its last size, one key past it (three launches), block edges and short ragged sequences.
+@pytest.mark.parametrize("case", [
+    (1, 2, 64, ROPE_HALF, True, True, False), (256, 2, 128, ROPE_INTERLEAVED, True, True, True),
+    (513, 3, 64, ROPE_HALF, True, True, False), (8192, 1, 64, ROPE_HALF, True, True, True),
+    (8193, 1, 128, ROPE_INTERLEAVED, True, True, False), (9001, 2, 0, ROPE_NONE, True, True, True),
+], ids=lambda c: f"S{c[0]}H{c[1]}r{c[2]}m{c[3]}")
+def test_norm_rope_prologue_lengths(cuda, case):
+    test_fused_norm_rope_prologue_is_bit_exact(cuda, case)
+
+
+def test_norm_rope_prologue_paths_agree(cuda):
+    """The one-pass prologue, its recompute path (the wait bounded to one look, so that
+    work-groups compute partials of other blocks from memory) and the three launches of a
+    captured call fill the workspace alike."""
+    from miroxen_amd import AttnParams, _lib, flash_attn_fp8_workspace, sage_layout, sage_quantize_norm_rope
+    S, H, D, rot = 3000, 4, 128, 64
+    print(f"norm/rope prologue paths S={S} H={H}", flush=True)
+    HD = H * D
+    g = torch.Generator(device=cuda).manual_seed(11)
+    t = (torch.randn(S, 3 * HD, device=cuda, generator=g) * 1.5).to(torch.bfloat16)
+    qw, kw = (torch.rand(D, device=cuda, generator=g) + 0.5 for _ in range(2))
+    ang = torch.rand(S, rot // 2, device=cuda, generator=g) * 6
+    cs, sn = ang.cos(), ang.sin()
+    p = AttnParams(Sq=S, Skv=S, Hq=H, Hkv=H, D=D, q_stride=3 * HD, kv_stride=3 * HD, o_stride=HD)
+    L, base = sage_layout(p), t.data_ptr()
+
+    def run(ws):
+        sage_quantize_norm_rope(base, base + 2 * HD, base + 4 * HD, p, qw, kw, 1e-6, cs, sn, rot, ROPE_HALF, ws)
+
+    def regions(ws):
+        torch.cuda.synchronize()
+        sizes = (("qi", H * L["sq_pad"] * D), ("ki", H * L["skv_pad"] * D), ("vt", H * D * L["skv_pad"]),
+                 ("qs", H * L["sq_pad"] // 4), ("ks", H * L["skv_pad"] // 16), ("km", 4 * HD), ("va", 4 * HD))
+        return {n: ws[L[n]: L[n] + b].clone() for n, b in sizes}
+
+    new = lambda: torch.full((flash_attn_fp8_workspace(p),), 0xA5, dtype=torch.uint8, device=cuda)
+    ws = new()
+    run(ws)
+    want = regions(ws)
+    lib = _lib.load()
+    _lib.check(lib.mx_sage_prologue_wait_ticks(0))
+    try:
+        for _ in range(3):
+            ws = new()
+            run(ws)
+            for n, x in regions(ws).items():
+                assert torch.equal(x, want[n]), f"recompute: {n}"
+    finally:
+        _lib.check(lib.mx_sage_prologue_wait_ticks(20000))
+    ws, other = new(), new()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(ws)
+    for i in range(3):
+        ws.fill_(0x5A)
+        graph.replay()
+        for n, x in regions(ws).items():
+            assert torch.equal(x, want[n]), f"replay {i}: {n}"
+        run(other)  # eager work between replays
+        torch.cuda.synchronize()
