@@ -26,7 +26,7 @@ namespace {
 // ---------------- prologue ----------------
 //
 // Eager calls with Skv <= 8192 run prep_kv_fused, one launch over K
-// and V (below), plus prep_stats_q's Q blocks when Q is quantized here. Otherwise
+// and V (below) whose last work-groups quantize Q when Q is quantized here. Otherwise
 // three launches (the reference uses a memset and four kernels, :433-446):
 //  1. prep_stats_q: blocks [0, Hkv*nb) reduce K/V statistics of one 256-token
 //     block of one head; the remaining blocks quantize Q (one 16-row group per
@@ -55,6 +55,54 @@ __device__ __forceinline__ u32x2 quant8(const float (&x)[8], float inv) {
 
 constexpr int kStatChunk = 128;  // tokens staged in LDS per step of a stats block
 constexpr int kFoldNb = 32;       // statistics partials per head up to which prep_kv_quant finalizes them
+
+// Quantization of Q by work-group blk of `waves` waves: one 16-row group per wave. QG = 64
+// needs four waves per work-group.
+template <int D, int NRM, int QG>
+__device__ __forceinline__ void quant_q(const uint16_t* __restrict__ q, const mx_attn_params& p, int64_t blk, int waves,
+                                        float qmult, int64_t sq_pad, int8_t* __restrict__ qi, float* __restrict__ qs,
+                                        const NormRope& nq) {
+  // a lane owns D / 32 chunks of 8 channels
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t gid = blk * waves + wave;  // group index over (head, group)
+  const int ng = int(sq_pad / 16);
+  if (gid >= int64_t(p.Hq) * ng) return;
+  const int h = int(gid / ng), grp = int(gid % ng);
+  constexpr int NCH = D / 32, CPR = D / 8;  // chunks per lane, chunks per row
+  float x[NCH][8], am = 0.f;
+  u32x4 raw[NCH];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int ci = lane + i * 64, r = ci / CPR, c = (ci % CPR) * 8;
+    const int64_t row = int64_t(grp) * 16 + r;
+    raw[i] = u32x4{0, 0, 0, 0};
+    if (row < p.Sq) raw[i] = *reinterpret_cast<const u32x4*>(q + row * p.q_stride + int64_t(h) * D + c);
+  }
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int64_t row = int64_t(grp) * 16 + (lane + i * 64) / CPR;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[i][j] = bf2f(uint16_t(raw[i][j >> 1] >> ((j & 1) * 16)));
+    // row r of the group on lanes 16(r&3) .. +15: the 16-lane layout of nr128_row
+    if constexpr (NRM >= 0) nr128_row<NRM>(x[i], row, row < p.Sq, nq, lane);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) am = fmaxf(am, fabsf(x[i][j]));
+  }
+  am = wave_max(am);
+  if constexpr (QG == 64) {  // the work-group's four waves hold the 64-row block
+    __shared__ float wmax[4];
+    if (lane == 0) wmax[wave] = am;
+    __syncthreads();
+    am = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+  }
+  const float inv = am > 0.f ? 127.f / am : 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int ci = lane + i * 64, r = ci / CPR, c = (ci % CPR) * 8;
+    *reinterpret_cast<u32x2*>(qi + (int64_t(h) * sq_pad + int64_t(grp) * 16 + r) * D + c) = quant8(x[i], inv);
+  }
+  if (lane == 0) qs[int64_t(h) * (sq_pad / 16) + grp] = am / 127.f * qmult;
+}
 
 // NRM >= 0: q and k are the raw projections; every row gets the per-head RMS-norm
 // + RoPE of head_norm_rope (nq / nk, nr128_row with rope mode NRM) and its bf16
@@ -131,46 +179,7 @@ __global__ void __launch_bounds__(256) prep_stats_q(const uint16_t* __restrict__
     else if (tid < 2 * D) part[int64_t(p.Hkv) * nb * D + (int64_t(h) * nb + b) * D + (tid - D)] = am;
     return;
   }
-  // ---- Q: one 16-row group per wave; lane owns D / 32 chunks of 8 channels ----
-  const int wave = tid >> 6, lane = tid & 63;
-  const int64_t gid = (int64_t(blockIdx.x) - nstat) * 4 + wave;  // group index over (head, group)
-  const int ng = int(sq_pad / 16);
-  if (gid >= int64_t(p.Hq) * ng) return;
-  const int h = int(gid / ng), grp = int(gid % ng);
-  constexpr int NCH = D / 32, CPR = D / 8;  // chunks per lane, chunks per row
-  float x[NCH][8], am = 0.f;
-  u32x4 raw[NCH];
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int ci = lane + i * 64, r = ci / CPR, c = (ci % CPR) * 8;
-    const int64_t row = int64_t(grp) * 16 + r;
-    raw[i] = u32x4{0, 0, 0, 0};
-    if (row < p.Sq) raw[i] = *reinterpret_cast<const u32x4*>(q + row * p.q_stride + int64_t(h) * D + c);
-  }
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int64_t row = int64_t(grp) * 16 + (lane + i * 64) / CPR;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[i][j] = bf2f(uint16_t(raw[i][j >> 1] >> ((j & 1) * 16)));
-    // row r of the group on lanes 16(r&3) .. +15: the 16-lane layout of nr128_row
-    if constexpr (NRM >= 0) nr128_row<NRM>(x[i], row, row < p.Sq, nq, lane);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) am = fmaxf(am, fabsf(x[i][j]));
-  }
-  am = wave_max(am);
-  if constexpr (QG == 64) {  // the work-group's four waves hold the 64-row block
-    __shared__ float wmax[4];
-    if (lane == 0) wmax[wave] = am;
-    __syncthreads();
-    am = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  }
-  const float inv = am > 0.f ? 127.f / am : 0.f;
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int ci = lane + i * 64, r = ci / CPR, c = (ci % CPR) * 8;
-    *reinterpret_cast<u32x2*>(qi + (int64_t(h) * sq_pad + int64_t(grp) * 16 + r) * D + c) = quant8(x[i], inv);
-  }
-  if (lane == 0) qs[int64_t(h) * (sq_pad / 16) + grp] = am / 127.f * qmult;
+  quant_q<D, NRM, QG>(q, p, int64_t(blockIdx.x) - nstat, 4, qmult, sq_pad, qi, qs, nq);
 }
 
 // kmean / vamax of one head from the statistics partials: the sum in ascending
@@ -500,7 +509,9 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
                                                      float* __restrict__ ks, uint8_t* __restrict__ vt,
                                                      u32x4* __restrict__ tab, int* __restrict__ cnt, int ncnt,
                                                      uint64_t* __restrict__ flg, uint64_t epoch, uint64_t wait_ticks,
-                                                     NormRope nk) {
+                                                     NormRope nk, const uint16_t* __restrict__ q, float qmult,
+                                                     int64_t sq_pad, int8_t* __restrict__ qi, float* __restrict__ qs,
+                                                     NormRope nq) {
   static_assert(D == 64 || D == 128, "head dimension 64 or 128");
   static_assert(NRM < 0 || D == 128, "the fused norm/rope prologue is built for D = 128");
   constexpr int NT = 512, CPR = D / 8, RPT = kStatTok * CPR / NT;  // chunks per row, tokens per thread
@@ -516,6 +527,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   __shared__ float red[NT / 64][D];
   __shared__ float kms[D], vas[D];
   __shared__ bool miss[kFoldNb];
+  // work-groups past the K/V blocks quantize Q: they fill the CUs while the last K/V blocks
+  // wait for their head and store (norm/RoPE prologue, 24 heads: x 1000 24.4 -> 20.3 us, x 4352
+  // 56 -> 47 against a launch of their own)
+  if (int(blockIdx.x) >= p.Hkv * nb) {
+    quant_q<D, NRM, 16>(q, p, int64_t(blockIdx.x) - int64_t(p.Hkv) * nb, NT / 64, qmult, sq_pad, qi, qs, nq);
+    return;
+  }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int h = blockIdx.x / nb, b = blockIdx.x % nb;
   const int c = tid % CPR, r0 = (tid / CPR) * RPT;
@@ -1635,16 +1653,22 @@ hipError_t sage_quantize_d(const uint16_t* q, const uint16_t* k, const uint16_t*
     const hipError_t ce = hipStreamIsCapturing(s, &cap);
     if (ce != hipSuccess) return ce;
     if (cap == hipStreamCaptureStatusNone) {
-      hipLaunchKernelGGL(fused, dim3(unsigned(int64_t(p.Hkv) * nb)), dim3(512), 0, s, k, v, p, nb,
-                         L.skv_pad, part, km, va, reinterpret_cast<int8_t*>(ws + L.ki),
-                         reinterpret_cast<float*>(ws + L.ks), reinterpret_cast<uint8_t*>(ws + L.vt),
-                         reinterpret_cast<u32x4*>(ws + L.tab), reinterpret_cast<int*>(ws + L.cnt), L.split_units,
-                         reinterpret_cast<uint64_t*>(ws + L.flg), next_epoch(),
-                         g_fused_wait_ticks.load(std::memory_order_relaxed), nk);
-      if (!skip_q && qgroups > 0)  // Q blocks only (no statistics blocks: nb = 0)
-        hipLaunchKernelGGL(stats, dim3(unsigned((qgroups + 3) / 4)), dim3(256), 0, s, q, k, v, p, 0, qmult,
-                           L.sq_pad, part, reinterpret_cast<int8_t*>(ws + L.qi), reinterpret_cast<float*>(ws + L.qs),
-                           nq, nk);
+      // Q's work-groups (8 groups of 16 rows each) follow K/V's in the same launch; Q scales
+      // per 64 rows are a launch of their own
+      const bool q16 = !skip_q && q_group != 64, q64 = !skip_q && q_group == 64;
+      const int64_t kvb = int64_t(p.Hkv) * nb, fb = kvb + (q16 ? (qgroups + 7) / 8 : 0);
+      if (fb > 0x7fffffff) return hipErrorInvalidValue;
+      int8_t* qi = reinterpret_cast<int8_t*>(ws + L.qi);
+      float* qs = reinterpret_cast<float*>(ws + L.qs);
+      hipLaunchKernelGGL(fused, dim3(unsigned(fb)), dim3(512), 0, s, k, v, p, nb, L.skv_pad, part, km, va,
+                         reinterpret_cast<int8_t*>(ws + L.ki), reinterpret_cast<float*>(ws + L.ks),
+                         reinterpret_cast<uint8_t*>(ws + L.vt), reinterpret_cast<u32x4*>(ws + L.tab),
+                         reinterpret_cast<int*>(ws + L.cnt), L.split_units, reinterpret_cast<uint64_t*>(ws + L.flg),
+                         next_epoch(), g_fused_wait_ticks.load(std::memory_order_relaxed), nk, q, qmult, L.sq_pad, qi,
+                         qs, nq);
+      if (q64 && qgroups > 0)  // Q blocks only (no statistics blocks: nb = 0)
+        hipLaunchKernelGGL(stats, dim3(unsigned((qgroups + 3) / 4)), dim3(256), 0, s, q, k, v, p, 0, qmult, L.sq_pad,
+                           part, qi, qs, nq, nk);
       return hipGetLastError();
     }
   }
