@@ -19,8 +19,8 @@
 // 4-wave work-group, one wave per SIMD, each wave 128 n x 128 m = 4 x 4 MFMA blocks
 // of 32 x 32 (C = W X^T: lane = one m column, 16 n rows; the 256 fp32 accumulators
 // live in AGPRs). K advances in stages of 128 bytes DMA'd into LDS
-// (buffer_load ... lds, 1 KB per op, rows past the matrix read as zeros), double
-// buffered; LDS rows are 128 B with their 16-byte chunks XOR'd by (row >> 1) & 7, so
+// (buffer_load ... lds, 1 KB per op, rows past the matrix read as zeros), in a ring of
+// slots; LDS rows are 128 B with their 16-byte chunks XOR'd by (row >> 1) & 7, so
 // each 16-lane group of an operand read hits 16 distinct chunk slots. A stage's
 // scales for a lane are one 16-byte load per operand (the interleave puts a 128-row
 // band's four 32-row blocks side by side). The bf16 tile leaves through LDS as
