@@ -363,11 +363,16 @@ __global__ void __launch_bounds__(256) prep_kv_quant(const uint16_t* __restrict_
 // K mean and V abs-max are known, and quantizes the block from its registers.
 // Same arithmetic as the three-launch path (bit-identical workspace).
 //
-// Flags: ws.flg holds one 64-bit word per (head, block); a word is
-// "set" when it equals the call's epoch, a per-process counter that never repeats
-// (and is never 0), so no flag needs clearing before a call and a workspace reused
-// across calls cannot satisfy a wait with an old flag. The host runs this path only
-// outside stream capture: a captured launch would replay with one fixed epoch.
+// Flags: ws.flg holds one 64-bit word per (head, block): the call's epoch, a per-process
+// counter that never repeats (a multiple of 4, never 0), with bit 0 set once the block's K
+// partial is out and bit 1 for its V partial. So no flag needs clearing before a call and a
+// workspace reused across calls cannot satisfy a wait with an old flag. The host runs this
+// path only outside stream capture: a captured launch would replay with one fixed epoch.
+//
+// SIDES = 2: K and V of a block are two work-groups, 2 (h nb + b) and the next; they share
+// nothing but the flag word (K's mean needs only K, V's scales only V). For grids that leave
+// CUs idle, where a work-group's own chain (load, sum, quantize: instruction-bound with both
+// tensors on one CU) is the call; see fused_sides for where.
 //
 // Waiting: work-groups are dispatched in index order and a head's blocks are
 // consecutive, so a head's blocks all get a slot while earlier heads drain (a head
@@ -394,14 +399,20 @@ __device__ __forceinline__ void st_dev(float* p, float x) {
   __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// True when flags f[0..n) all equal epoch; false once `ticks` of the chip clock have
+// Whether flag word f says that the partials of `need` (bit 0: K, bit 1: V) are out.
+__device__ __forceinline__ bool flag_set(const uint64_t* f, uint64_t epoch, uint32_t need) {
+  return (__hip_atomic_load(const_cast<uint64_t*>(f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | (3u ^ need)) ==
+         (epoch | 3u);
+}
+
+// True when flags f[0..n) are all set (flag_set); false once `ticks` of the chip clock have
 // passed (ticks 0: one look). Work-group uniform; every thread must call it.
-__device__ __forceinline__ bool wait_flags(const uint64_t* f, int n, uint64_t epoch, uint64_t ticks) {
+__device__ __forceinline__ bool wait_flags(const uint64_t* f, int n, uint64_t epoch, uint32_t need,
+                                           uint64_t ticks) {
   const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
   for (;;) {
     bool ok = true;
-    for (int j = threadIdx.x; j < n; j += blockDim.x)
-      ok &= __hip_atomic_load(const_cast<uint64_t*>(f + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch;
+    for (int j = threadIdx.x; j < n; j += blockDim.x) ok &= flag_set(f + j, epoch, need);
     if (__syncthreads_and(ok)) return true;
     const bool late = threadIdx.x == 0 && __builtin_amdgcn_s_memrealtime() - t0 >= ticks;
     if (__syncthreads_or(late)) return false;
@@ -447,16 +458,15 @@ __device__ void fused_stats_from_memory(const uint16_t* __restrict__ k, const ui
 }
 
 // Wait for every block flag of head h (bounded), compute the partials still missing,
-// and return this thread's channel of K mean / V abs-max (threads < D) summed in
-// ascending block order (finalize_channel's arithmetic on device-scope loads).
+// and return this thread's channel of K mean / V abs-max (threads < D; the one that `need`
+// names) summed in ascending block order (finalize_channel's arithmetic on device-scope loads).
 template <int D, int NRM>
 __device__ void fused_fold(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const mx_attn_params& p,
-                           const NormRope& nk, int h, int nb, float* part, const uint64_t* flg, uint64_t epoch, uint64_t ticks,
+                           const NormRope& nk, int h, int nb, float* part, const uint64_t* flg, uint64_t epoch, uint32_t need, uint64_t ticks,
                            unsigned char* sm, bool* miss, float& s, float& am) {
   const uint64_t* fh = flg + int64_t(h) * nb;
-  if (!wait_flags(fh, nb, epoch, ticks)) {
-    for (int j = threadIdx.x; j < nb; j += blockDim.x)
-      miss[j] = __hip_atomic_load(const_cast<uint64_t*>(fh + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch;
+  if (!wait_flags(fh, nb, epoch, need, ticks)) {
+    for (int j = threadIdx.x; j < nb; j += blockDim.x) miss[j] = !flag_set(fh + j, epoch, need);
     __syncthreads();
     for (int j = 0; j < nb; ++j)
       if (miss[j]) fused_stats_from_memory<D, NRM>(k, v, p, nk, h, j, nb, part, sm);
@@ -501,7 +511,7 @@ __device__ void fused_fold(const uint16_t* __restrict__ k, const uint16_t* __res
 // One work-group of 512 threads per (head, 256-token block): thread t owns channel
 // chunk c = t % (D/8) (8 channels) of the RPT consecutive tokens from (t / (D/8)) RPT.
 // NRM >= 0: K rows get norm and RoPE (nk) in registers before anything else is done with them.
-template <int D, int NRM>
+template <int D, int NRM, int SIDES>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) prep_kv_fused(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                      mx_attn_params p, int nb, int64_t skv_pad,
                                                      float* __restrict__ part, float* __restrict__ km,
@@ -530,12 +540,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   // work-groups past the K/V blocks quantize Q: they fill the CUs while the last K/V blocks
   // wait for their head and store (norm/RoPE prologue, 24 heads: x 1000 24.4 -> 20.3 us, x 4352
   // 56 -> 47 against a launch of their own)
-  if (int(blockIdx.x) >= p.Hkv * nb) {
-    quant_q<D, NRM, 16>(q, p, int64_t(blockIdx.x) - int64_t(p.Hkv) * nb, NT / 64, qmult, sq_pad, qi, qs, nq);
+  const int nkv = SIDES * p.Hkv * nb;
+  if (int(blockIdx.x) >= nkv) {
+    quant_q<D, NRM, 16>(q, p, int64_t(blockIdx.x) - nkv, NT / 64, qmult, sq_pad, qi, qs, nq);
     return;
   }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int h = blockIdx.x / nb, b = blockIdx.x % nb;
+  const int hb = int(blockIdx.x) / SIDES, h = hb / nb, b = hb % nb;
+  const bool do_k = SIDES == 1 || !(blockIdx.x & 1), do_v = SIDES == 1 || (blockIdx.x & 1);
+  const uint32_t need = (do_k ? 1u : 0u) | (do_v ? 2u : 0u);
   const int c = tid % CPR, r0 = (tid / CPR) * RPT;
   const int64_t t0 = int64_t(b) * kStatTok;
   const int rows = int(p.Skv - t0 < kStatTok ? p.Skv - t0 : kStatTok);
@@ -547,15 +560,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
     kr[i] = vr[i] = u32x4{0, 0, 0, 0};
     if (r0 + i < rows) {
       const int64_t g = (t0 + r0 + i) * p.kv_stride + int64_t(h) * D + c * 8;
-      kr[i] = *reinterpret_cast<const u32x4*>(k + g);
-      vr[i] = *reinterpret_cast<const u32x4*>(v + g);
+      if (do_k) kr[i] = *reinterpret_cast<const u32x4*>(k + g);
+      if (do_v) vr[i] = *reinterpret_cast<const u32x4*>(v + g);
     }
   }
   if (blockIdx.x == 0)  // arrival counters of the attention kernel's split units start at zero
     for (int i = tid; i < ncnt; i += NT) cnt[i] = 0;
   if constexpr (NRM >= 0) {
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {  // (rows past Skv stay zeros)
+    for (int i = 0; i < RPT && do_k; ++i) {  // (rows past Skv stay zeros)
       nr128_words<NRM>(kr[i], t0 + r0 + i, r0 + i < rows, nk, lane);
       if (r0 + i >= rows) kr[i] = u32x4{0, 0, 0, 0};
       if (i & 1) __builtin_amdgcn_sched_barrier(0);  // two rows at a time: all eight at once spill
@@ -569,7 +582,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   // chunk per pass, and for the sum's reads, 16 channels' same chunk), so the sum reads
   // 8 tokens per LDS read; D = 64: token-major [256][D]
   uint16_t* kst = reinterpret_cast<uint16_t*>(sm);
-  if constexpr (D == 128) {
+  if (!do_k) {
+  } else if constexpr (D == 128) {
 #pragma unroll
     for (int j2 = 0; j2 < 4; ++j2)
 #pragma unroll
@@ -590,7 +604,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   using u16x2 = __attribute__((ext_vector_type(2))) unsigned short;
   u16x2 vam[4];
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < 4 && do_v; ++w) {
     vam[w] = u16x2{0, 0};
 #pragma unroll
     for (int i = 0; i < RPT; ++i)
@@ -600,12 +614,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
       vam[w] = __builtin_elementwise_max(
           vam[w], __builtin_bit_cast(u16x2, uint32_t(__shfl_xor(int(__builtin_bit_cast(uint32_t, vam[w])), off))));
   }
-  if (lane < CPR)
+  if (do_v && lane < CPR)
 #pragma unroll
     for (int j = 0; j < 8; ++j) red[wave][c * 8 + j] = bf2f(vam[j >> 1][j & 1]);
   __syncthreads();
   MX_STAMP(1);
-  if (tid < D) {
+  if (do_k && tid < D) {
     float sum = 0.f;
     if constexpr (D == 128) {  // tokens past the block's end are zeros: adding +0 changes no sum
                                // (a sum from +0 is never -0)
@@ -621,7 +635,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
       for (int r = 0; r < rows; ++r) sum += bf2f(kst[r * D + tid]);  // sequential, token order
     }
     st_dev(part + (int64_t(h) * nb + b) * D + tid, sum / float(p.Skv));
-  } else if (tid < 2 * D) {
+  } else if (do_v && tid >= D && tid < 2 * D) {
     float am = 0.f;
 #pragma unroll
     for (int w = 0; w < NT / 64; ++w) am = fmaxf(am, red[w][tid - D]);
@@ -629,16 +643,25 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   }
   wait_vm();
   __syncthreads();
-  if (tid == 0)
-    __hip_atomic_store(flg + int64_t(h) * nb + b, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) {
+    uint64_t* f = flg + int64_t(h) * nb + b;
+    if constexpr (SIDES == 1) {
+      __hip_atomic_store(f, epoch | 3u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {  // keep the other side's bit if it is this call's (one other writer: at most two turns)
+      uint64_t old = __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      while (!__hip_atomic_compare_exchange_strong(f, &old, ((old & ~uint64_t(3)) == epoch ? old : epoch) | need,
+                                                   __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      }
+    }
+  }
   MX_STAMP(2);
 
   // ---- K mean and V abs-max of the head: every work-group folds the partials ----
   float s = 0.f, am = 0.f;
-  fused_fold<D, NRM>(k, v, p, nk, h, nb, part, flg, epoch, wait_ticks, sm, miss, s, am);
+  fused_fold<D, NRM>(k, v, p, nk, h, nb, part, flg, epoch, need, wait_ticks, sm, miss, s, am);
   if (b == 0 && tid < D) {
-    km[h * D + tid] = s;
-    va[h * D + tid] = am;
+    if (do_k) km[h * D + tid] = s;
+    if (do_v) va[h * D + tid] = am;
   }
   if (tid < D) {
     kms[tid] = s;
@@ -669,16 +692,18 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
       for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(kx(i, j, fullc)));
     return m;
   };
-  float tam = full ? k_amax(std::true_type{}) : k_amax(std::false_type{});
-  tam = wave_max(tam);
+  float tam = 0.f;
   float* tred = &red[0][0];
-  if (lane == 0) tred[wave] = tam;
+  if (do_k) {
+    tam = wave_max(full ? k_amax(std::true_type{}) : k_amax(std::false_type{}));
+    if (lane == 0) tred[wave] = tam;
+  }
 
   // ---- V -> e4m3 into the V^T tile in LDS: channel row d, RPT-byte granule of
   // tokens r0.. at granule (r0 / RPT) ^ vsw(c), which spreads a wave's
   // writes over every bank ----
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < 8 && do_v; ++j) {
     // rows past Skv are zeros (0 * vsc = +0); a channel with no nonzero value stays 0
     float f[RPT];
     const bool live = vsc[j] > 0.f;
@@ -698,7 +723,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   __syncthreads();
   tam = fmaxf(tred[2 * tl], tred[2 * tl + 1]);
   const float inv = tam > 0.f ? 127.f / tam : 0.f;
-  if (key0 < skv_pad) {
+  if (do_k && key0 < skv_pad) {
     auto k_store = [&](auto fullc) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < RPT; ++i) {
@@ -724,7 +749,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   }
   // ---- V^T rows: channel d, the block's keys below skv_pad, 16 bytes per thread ----
   const int nkeys = int(skv_pad - t0 < kStatTok ? skv_pad - t0 : kStatTok);
-  for (int i = tid; i < D * (kStatTok / 16); i += NT) {
+  for (int i = tid; do_v && i < D * (kStatTok / 16); i += NT) {
     const int d = i / (kStatTok / 16), u = i % (kStatTok / 16);
     if (u * 16 >= nkeys) continue;
     const int gi = (u * (16 / RPT)) ^ vsw(d >> 3);
@@ -1552,8 +1577,8 @@ SagePlan sage_plan(const mx_attn_params& p) {
   return pl;
 }
 
-// Epoch of one fused-prologue call: a per-process counter from a random start, never 0
-// (a zeroed workspace holds no set flag).
+// Epoch of one fused-prologue call: a per-process counter from a random start, a multiple of 4,
+// never 0 (a zeroed workspace holds no set flag).
 uint64_t next_epoch() {
   static std::atomic<uint64_t> ctr{[] {
     uint64_t x = uint64_t(std::chrono::steady_clock::now().time_since_epoch().count()) * 0x9E3779B97F4A7C15ull;
@@ -1562,12 +1587,21 @@ uint64_t next_epoch() {
       x ^= (uint64_t(rd()) << 32) ^ uint64_t(rd());
     } catch (...) {
     }
-    return x;
+    return x & ~uint64_t(3);
   }()};
   uint64_t e;
-  do e = ctr.fetch_add(1, std::memory_order_relaxed);
+  do e = ctr.fetch_add(4, std::memory_order_relaxed);
   while (e == 0);
   return e;
+}
+
+// Work-groups per (head, 256-token block) of the one-pass prologue: K and V apart while every
+// half still gets a CU of its own (256). Call us, one / two: 24 heads x 256 keys 21.1 / 19.3,
+// x 600 26.7 / 25.3, x 1088 (120 blocks) 33.0 / 31.3, 8 x 4096 (128) 64.6 / 62.5; with norm/RoPE
+// 25.4 / 22.4, 32.2 / 29.1, 39.9 / 36.3, 70.2 / 66.6. Beyond, the halves queue for the same
+// CUs and gain nothing or lose: 24 x 1500 (144) 49.5 / 49.5 and 55.3 / 56.5, x 4352 181 / 186.
+int fused_sides(int64_t blocks) {
+  return blocks <= 128 ? 2 : 1;
 }
 
 mx_sage_layout sage_layout(const mx_attn_params& p) {
@@ -1627,20 +1661,27 @@ hipError_t sage_quantize_d(const uint16_t* q, const uint16_t* k, const uint16_t*
   static_assert(kSqPad % 64 == 0, "Q padding must cover whole 64-row blocks");
   decltype(&prep_stats_q<D, -1, 16>) stats;
   decltype(&prep_kv_quant<D, -1>) kvq;
-  decltype(&prep_kv_fused<D, -1>) fused;
+  decltype(&prep_kv_fused<D, -1, 1>) fused;
+  const int sides = fused_sides(int64_t(p.Hkv) * nb);
+  auto pick = [&](auto nrm) {
+    constexpr int N = decltype(nrm)::value;
+    return sides == 2 ? prep_kv_fused<D, N, 2> : prep_kv_fused<D, N, 1>;
+  };
   if constexpr (D == 128) {
     stats = q_group == 64 ? prep_stats_q<D, -1, 64>
           : mode < 0 ? prep_stats_q<D, -1, 16> : mode == kRopeNone ? prep_stats_q<D, kRopeNone, 16>
           : mode == kRopeInterleaved ? prep_stats_q<D, kRopeInterleaved, 16> : prep_stats_q<D, kRopeHalf, 16>;
     kvq = mode < 0 ? prep_kv_quant<D, -1> : mode == kRopeNone ? prep_kv_quant<D, kRopeNone>
         : mode == kRopeInterleaved ? prep_kv_quant<D, kRopeInterleaved> : prep_kv_quant<D, kRopeHalf>;
-    fused = mode < 0 ? prep_kv_fused<D, -1> : mode == kRopeNone ? prep_kv_fused<D, kRopeNone>
-          : mode == kRopeInterleaved ? prep_kv_fused<D, kRopeInterleaved> : prep_kv_fused<D, kRopeHalf>;
+    fused = mode < 0 ? pick(std::integral_constant<int, -1>{})
+          : mode == kRopeNone ? pick(std::integral_constant<int, kRopeNone>{})
+          : mode == kRopeInterleaved ? pick(std::integral_constant<int, kRopeInterleaved>{})
+          : pick(std::integral_constant<int, kRopeHalf>{});
   } else {
     if (mode >= 0) return hipErrorInvalidValue;  // the fused norm/rope prologue is D = 128 only
     stats = q_group == 64 ? prep_stats_q<D, -1, 64> : prep_stats_q<D, -1, 16>;
     kvq = prep_kv_quant<D, -1>;
-    fused = prep_kv_fused<D, -1>;
+    fused = pick(std::integral_constant<int, -1>{});
   }
   // one-pass K/V prologue (prep_kv_fused) outside stream capture
 #ifdef MX_STAMPS
@@ -1656,7 +1697,7 @@ hipError_t sage_quantize_d(const uint16_t* q, const uint16_t* k, const uint16_t*
       // Q's work-groups (8 groups of 16 rows each) follow K/V's in the same launch; Q scales
       // per 64 rows are a launch of their own
       const bool q16 = !skip_q && q_group != 64, q64 = !skip_q && q_group == 64;
-      const int64_t kvb = int64_t(p.Hkv) * nb, fb = kvb + (q16 ? (qgroups + 7) / 8 : 0);
+      const int64_t kvb = int64_t(p.Hkv) * nb * sides, fb = kvb + (q16 ? (qgroups + 7) / 8 : 0);
       if (fb > 0x7fffffff) return hipErrorInvalidValue;
       int8_t* qi = reinterpret_cast<int8_t*>(ws + L.qi);
       float* qs = reinterpret_cast<float*>(ws + L.qs);

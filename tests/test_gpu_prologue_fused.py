@@ -150,6 +150,40 @@ def test_fused_prologue_recompute_path(cuda):
         _lib.check(lib.mx_sage_prologue_wait_ticks(20000))
 
 
+# Up to 128 (head, block) pairs K and V of a block are two work-groups that share one flag word:
+# both sides of that line, at whole and ragged blocks, D = 64 and 128, and with the bounded
+# wait forced to one look (each side recomputes the partials it has not seen).
+# Skv, H, D, forced
+SIDES = [(1024, 32, 128, False), (513, 43, 128, False), (1, 128, 128, False), (300, 64, 64, False),
+         (2048, 16, 128, True), (600, 40, 64, True), (2100, 15, 128, True)]
+
+
+@pytest.mark.parametrize("case", SIDES, ids=lambda c: "x".join(map(str, c)))
+def test_fused_prologue_k_and_v_apart(cuda, case):
+    from miroxen_amd import _lib
+    Skv, H, D, forced = case
+    print(f"K and V work-groups {case}", flush=True)
+    q, k, v, qs, ks = _bias_inputs(33, Skv, H, H, D, 0, 4.0, cuda, Skv + H)
+    p = AttnParams(Sq=33, Skv=Skv, Hq=H, Hkv=H, D=D)
+    L = sage_layout(p)
+    ws = _ws(p, cuda)
+    ws.fill_(0xFF)
+    _, want = oracle.sage_reference(_bits(q), _bits(k), _bits(v), 33, Skv, H, H, D, q_stride=qs, kv_stride=ks,
+                                    rows=np.zeros(0, np.int32))
+    lib = _lib.load()
+    if forced:
+        _lib.check(lib.mx_sage_prologue_wait_ticks(0))
+    try:
+        for _ in range(3):  # (old flags of the call before in place)
+            sage_quantize(q, k, v, p, ws)
+            torch.cuda.synchronize()
+            got = _quantized(ws, p, L)
+            for name in REGIONS:
+                assert np.array_equal(got[name], want[name]), f"{name} differs from the reference quantizer"
+    finally:
+        _lib.check(lib.mx_sage_prologue_wait_ticks(20000))
+
+
 def _random_cases(n, seed):
     rng = np.random.default_rng(seed)
     out = []
