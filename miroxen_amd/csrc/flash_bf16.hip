@@ -663,12 +663,28 @@ flash_bf16_ks(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, co
   auto ld_v = [&](int t, unsigned char* d) __attribute__((always_inline)) {
     load_tile<4, true, DH>(v, t < nt ? t : nt - 1, d, p, kvbase, wq, ta);
   };
+  // The group's first K tile and Q are loaded first: the first scores need no more. Q's sign is
+  // applied behind the V tile's and the second K tile's ops, inside each branch, where the
+  // compiler knows how many ops may stay in flight; the asm keeps it there. Against one wait
+  // for all of them (us): 333 causal keys x 32 heads 12.3 -> 12.05, x 1000 22.0 -> 21.5,
+  // 24 heads x 2600 91.8 -> 90.8.
+  auto q_sign = [&](auto group) __attribute__((always_inline)) {
+#pragma unroll
+    for (int cc = 0; cc < A.NC; ++cc) {
+      asm volatile("; group %1" : "+v"(A.q[cc]) : "n"(decltype(group)::value));
+      A.q[cc] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, A.q[cc]) ^ qsign);
+    }
+  };
+  if (group_a) ld_k(0, ka0);
+  else ld_k(1, kb0);
+  qblock_init(A, q, p, q0, head, ln, 0);
   if (group_a) {
-    ld_k(0, ka0), ld_v(0, va0), ld_k(2, ka1);
+    ld_v(0, va0), ld_k(2, ka1);
+    q_sign(std::integral_constant<int, 0>{});
   } else {
-    ld_k(1, kb0), ld_v(1, vb0), ld_k(3, kb1);
+    ld_v(1, vb0), ld_k(3, kb1);
+    q_sign(std::integral_constant<int, 1>{});
   }
-  qblock_init(A, q, p, q0, head, ln, qsign);
   if (mask16) live16_finish<8>(live_tiles, lv16, p, nt, wave_u, ln.lane);
   else build_live<8, KT>(live_tiles, p, nt, wave, ln.lane);
 
@@ -692,8 +708,11 @@ flash_bf16_ks(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, co
     rescale(A);
   };
 
-  wait_vm_n<0>();
-  __syncthreads();  // the first tiles and the liveness bitmaps are visible
+  // the first K tile and the liveness bitmaps are visible (each wave has at least this many
+  // ops of the V tile and the second K tile behind its share of the first)
+  wait_vm_n<Dm::VOPS / 4 + Dm::KOPS / 4>();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  block_sync();
   if (group_a) {
     scores(ka0, A, ln);
     sched_k<2 * Dm::NC, 0>();
@@ -835,7 +854,7 @@ static __device__ __align__(256) unsigned char bf16_split_scratch[kBfSplitBytes]
 // Whether an unsplit call runs flash_bf16_ks (128-query units, key tiles alternating between
 // the wave groups) instead of flash_bf16_pp (256-query units). Causal: when the 256-query units
 // are one round or less, i.e. when the longest one sets the time (us, pp / ks; 32 query heads:
-// 333 keys 14.6 / 12.4, 1000 34 / 23, 2048 queries x 2165 keys 60.6 / 50.7, 12 heads x 3000
+// 333 keys 14.4 / 12.1, 1000 34 / 22, 2048 queries x 2165 keys 60.0 / 50.7, 12 heads x 3000
 // 68 / 47; beyond one round pp, 32 x 3000 86 / 94, 32 x 8192 504 / 555). Otherwise by the
 // estimates R (7 + 1.68 ceil(nt / 2)) and R' (6.5 + 1.37 nt) us in R and R' rounds of units,
 // the latter less 15 % where its last round is part of several (fewer busy CUs run at a higher
