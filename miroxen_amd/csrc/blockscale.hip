@@ -314,7 +314,6 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
   // on stage st's buffer is free and takes stage st + NBUF: its DMA op u goes into slot SL +
   // PRE + 5/8 * 2 SL * u / ND, the last ones into the first slots of stage st + 1.
   constexpr int SL = NI * NJ, PRE = SL >= 8 ? 2 : 1, ND = 2 * (NI + NJ), NP = 2 * (NI + NJ);
-  constexpr int SCL = 2;  // scale loads per stage
   auto dma_slot = [](int u) constexpr { return SL + PRE + u * 5 * SL / (4 * ND); };
   static_assert(dma_slot(ND - 1) < 3 * SL, "a stage's DMA ends before its wait");
   // DMA op u: operand u & 1 (X's ops run out first or last when NI != NJ), index u >> 1
@@ -409,7 +408,7 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
     }
   });
   if constexpr (NBUF > 2) {
-    wait_vm_n<(NBUF - 2) * (ND + SCL) + kEarly + SCL>();
+    wait_vm_n<(NBUF - 2) * ND + kEarly>();  // stage 0 landed (see the wait in `stage`)
     unpack(ra[0], rb[0], ta[0], tb[0]);
   }
   block_sync();
@@ -439,8 +438,11 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
       mm(S1{}, qc, r1a, r1b, ta[s], tb[s]);
       MXA_SCHED;
     });
-    // this wave's loads of stage st + 1 landed (newer: the stages up to st + NBUF - 1, touches) ...
-    wait_vm_n<(NBUF - 2) * (ND + SCL + TOUCH) + TOUCH>();
+    // this wave's DMA of stage st + 1 landed (newer: the stages up to st + NBUF - 1, a touch) ...
+    // Only LDS-DMA ops are counted. The two scale loads of a stage lie between them, but in the
+    // stages behind the loop over whole turns the compiler deletes those whose words nothing
+    // uses: counted in, they let that many DMA ops of stage st + 1 stay in flight.
+    wait_vm_n<(NBUF - 2) * ND + TOUCH>();
     block_sync();  // ... for every wave, and every wave has read stage st
     MXA_SCHED;
     static_for<SL - PRE>([&](auto qc) __attribute__((always_inline)) {

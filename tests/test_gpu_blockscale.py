@@ -187,6 +187,15 @@ def test_gemm_tile_kinds(cuda, M, N, K, pad, beta):
     _sampled_rows_match(QMode.MXFP8, M, N, K, pad, beta, cuda)
 
 
+# Every remainder of the K stages modulo the ring depth of the 256 x 128 (3 slots) and 128 x 128
+# (4 slots) tiles, behind at least one whole turn of the ring.
+@pytest.mark.parametrize("M,N,K", [(700, 5500, 128 * st - pad) for st, pad in ((7, 0), (8, 32), (9, 96))] +
+                         [(300, 7000, 128 * st - pad) for st, pad in ((7, 0), (8, 32), (9, 64), (10, 0), (11, 96))] +
+                         [(512, 5120, 896), (512, 5120, 3456)])
+def test_gemm_ring_remainders(cuda, M, N, K):
+    _sampled_rows_match(QMode.MXFP8, M, N, K, 0, 0.0, cuda)
+
+
 # ---------------- NVFP4 (reference blockscale.cu NVFP4 branch) ----------------
 
 def _quant4(x, rows, K, cuda, ldx=None):
