@@ -99,6 +99,11 @@ __device__ __forceinline__ void store_b128_sc1(u32x4 d, __amdgpu_buffer_rsrc_t r
 // LDS reads issued before the barrier have been consumed (their lgkmcnt waited)
 // before the barrier by construction.
 __device__ __forceinline__ void block_sync() { asm volatile("s_barrier" ::: "memory"); }
+// The same where that does not follow by construction: this wave's LDS reads have returned
+// (what they read may be overwritten behind the barrier) and its LDS writes are done.
+__device__ __forceinline__ void block_sync_lds() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
 
 // Key-liveness of one key per lane for a later tile: the in-range flag needs no
 // memory, the mask byte is loaded from a clamped index and only combined (in

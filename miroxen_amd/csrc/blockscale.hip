@@ -150,7 +150,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[NI][NJ], unsigned
   constexpr int CH = 8 * NI, RB = 16 * CH;  // chunks and bytes per row
   static_assert(NI == 2 || NI == 4, "rows of 256 or 512 bytes");
   const int n = lane & 31, h = lane >> 5;
-  block_sync();  // every wave is done with the operand buffers
+  block_sync_lds();  // every wave is done with the operand buffers
   {
     const int xs = n & 15;  // m % 16: wm and 32 j are multiples of 16
     unsigned char* wp = lds + (wm + n) * RB + 8 * h + wn * 2;
@@ -443,7 +443,9 @@ mxfp8_gemm(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, cons
     // stages behind the loop over whole turns the compiler deletes those whose words nothing
     // uses: counted in, they let that many DMA ops of stage st + 1 stay in flight.
     wait_vm_n<(NBUF - 2) * ND + TOUCH>();
-    block_sync();  // ... for every wave, and every wave has read stage st
+    // ... for every wave, and every wave has read stage st (the youngest operand reads were
+    // issued only PRE MFMAs ago: they are waited for here, the next DMA op goes into their slot)
+    block_sync_lds();
     MXA_SCHED;
     static_for<SL - PRE>([&](auto qc) __attribute__((always_inline)) {
       constexpr int q = decltype(qc)::value;

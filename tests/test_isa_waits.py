@@ -131,3 +131,33 @@ def test_ksplit_stage_landed_before_its_reads(kernels, f4, ni, nj, nb):
 @pytest.mark.parametrize("ni,nj", [(4, 4), (4, 2), (2, 2)])
 def test_nvfp4_stage_landed_at_its_barrier(kernels, ni, nj):
     assert max(_dma_in_flight(kernels["nvfp4_gemm", (ni, nj)], "s_barrier")) == 0
+
+
+def _lds_outstanding(body):
+    """For each s_barrier, in program order: the most LDS reads and writes that can be
+    outstanding there, over every path (LDS operations return in order)."""
+    blocks, worst, state, todo = _blocks(body), {}, {0: (0, 0)}, [0]
+    while todo:
+        b = todo.pop()
+        n, (code, to) = list(state[b]), blocks[b]
+        for i, s in enumerate(code):
+            if s.startswith("ds_"):
+                n[s.startswith("ds_write")] += 1
+            if s.startswith("s_waitcnt") and _count("lgkmcnt", s) is not None:
+                n = [min(x, _count("lgkmcnt", s)) for x in n]
+            if s.startswith("s_barrier"):
+                worst[b, i] = tuple(n)
+        for t in to:
+            old = state.get(t)
+            new = tuple(min(max(x), 64) for x in zip(n, old or n))
+            if new != old:
+                state[t] = new
+                todo.append(t)
+    return [worst[k] for k in sorted(worst)]
+
+
+def test_no_lds_read_outstanding_at_a_barrier(kernels):
+    """Behind a barrier a slot that was read is filled again, or takes the output tile."""
+    for name, body in kernels.items():
+        got = _lds_outstanding(body)
+        assert got and max(r for r, _ in got) == 0, (name, got)
