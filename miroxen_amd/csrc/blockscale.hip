@@ -182,7 +182,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[NI][NJ], unsigned
         }
       }
   }
-  block_sync();
+  block_sync_lds();  // the whole tile is written
   const bool vec = (reinterpret_cast<uintptr_t>(y) & 15) == 0 && ldy % 8 == 0;
 #pragma unroll 4
   for (int it = 0; it < 2 * NJ * NI; ++it) {

@@ -161,3 +161,10 @@ def test_no_lds_read_outstanding_at_a_barrier(kernels):
     for name, body in kernels.items():
         got = _lds_outstanding(body)
         assert got and max(r for r, _ in got) == 0, (name, got)
+
+
+def test_no_lds_write_outstanding_at_a_barrier(kernels):
+    """Behind a barrier other waves read what was written (output tile, partial tiles)."""
+    for name, body in kernels.items():
+        got = _lds_outstanding(body)
+        assert got and max(w for _, w in got) == 0, (name, got)
