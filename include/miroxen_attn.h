@@ -96,6 +96,10 @@ int mx_flash_attn_uses_mfma(const void* q, const void* k, const void* v, const v
  * are planned. Causal calls and calls under stream capture run unsplit. Launches
  * nothing. */
 int mx_flash_attn_split_plan(const mx_attn_params* p, int cus, int* full, int* units, int* parts);
+/* No counterpart in the reference (a diagnostic query): *queries = 128 when an eager
+ * mx_flash_attn call of these parameters runs whole in 128-query units, 256 otherwise;
+ * cus as above. Launches nothing. */
+int mx_flash_attn_unit_queries(const mx_attn_params* p, int cus, int* queries);
 
 /* No counterpart in the reference. For callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc):

@@ -104,6 +104,16 @@ def flash_attn_split_plan(p: AttnParams, cus: int = 0) -> tuple:
     return f.value, u.value, s.value
 
 
+def flash_attn_unit_queries(p: AttnParams, cus: int = 0) -> int:
+    """128 when an eager flash_attn call of this shape runs whole in 128-query units on a
+    device with `cus` compute units (0: the current device), else 256; a diagnostic query
+    with no counterpart in the reference."""
+    c = p.c()
+    n = ctypes.c_int(0)
+    _lib.check(_lib.load().mx_flash_attn_unit_queries(ctypes.byref(c), int(cus), ctypes.byref(n)))
+    return n.value
+
+
 def flash_attn_fp8_ok(q, k, v, o, p: AttnParams) -> bool:
     """Reference mx::flash_attn_fp8_ok (src/kernels/attention_fp8.cu:484-486)."""
     c = p.c()

@@ -855,7 +855,15 @@ static __device__ __align__(256) unsigned char bf16_split_scratch[kBfSplitBytes]
 // the wave groups) instead of flash_bf16_pp (256-query units). Causal: when the 256-query units
 // are one round or less, i.e. when the longest one sets the time (us, pp / ks; 32 query heads:
 // 333 keys 14.4 / 12.1, 1000 34 / 22, 2048 queries x 2165 keys 60.0 / 50.7, 12 heads x 3000
-// 68 / 47; beyond one round pp, 32 x 3000 86 / 94, 32 x 8192 504 / 555). Otherwise by the
+// 68 / 47; beyond one round pp, 32 x 3000 86 / 94, 32 x 8192 504 / 555), and either the 128-query
+// units are one round too (512 queries x 32 heads behind 8192 keys 181 / 108) or they differ in
+// length: two rounds of them gain by balance alone, and behind a long cache, where the first
+// query tile sees nearly as many keys as the last, they only add set-ups and K/V traffic. By
+// that share of keys: 2048 queries x 32 behind 1024 keys (0.38) 82 / 73, behind 4096 (0.69) 167 /
+// 164, behind 8192 (0.81) 278 / 283; 1500 x 32 behind 2048 (0.61) 84 / 80, 4096 (0.76) 130 / 131,
+// 8192 (0.86) 221 / 232; 2560 x 16 behind 4096 (0.64) 141 / 135, 8192 (0.77) 222 / 236; 1000 x 64
+// behind 1024 (0.57) 59.4 / 58.5, 2048 (0.71) 87.4 / 88.6, 8192 (0.91) 254 / 266: the line is at 0.7.
+// Otherwise (no causal mask) by the
 // estimates R (7 + 1.68 ceil(nt / 2)) and R' (6.5 + 1.37 nt) us in R and R' rounds of units,
 // the latter less 15 % where its last round is part of several (fewer busy CUs run at a higher
 // clock): 24 heads x 1088 28.7 / 21.5, x 2600 107 / 87, 16 heads of 72 x 2000 44 / 29, and pp
@@ -864,7 +872,13 @@ bool use_ks(const mx_attn_params& p, int C) {
   const int nt = (p.Skv + KT - 1) / KT;
   const int64_t U = int64_t((p.Sq + 255) / 256) * p.Hq, Uk = int64_t((p.Sq + 127) / 128) * p.Hq;
   if (C <= 0 || Uk > 0x7fffffff) return false;
-  if (p.causal) return U <= C && nt >= 3;
+  if (p.causal) {
+    auto keys = [&](int q) {  // visible to the queries before q
+      const int64_t n = int64_t(p.q_offset) + (q < p.Sq ? q : p.Sq);
+      return n < 0 ? 0 : n < p.Skv ? n : int64_t(p.Skv);
+    };
+    return U <= C && nt >= 3 && (Uk <= C || 10 * keys(128) <= 7 * keys(p.Sq));
+  }
   const double rounds = double((U + C - 1) / C), ks_rounds = double((Uk + C - 1) / C);
   const double pp = rounds * (6.5 + 1.37 * nt) * (rounds > 1 ? 0.85 : 1.0);
   return ks_rounds * (7.0 + 1.68 * ((nt + 1) / 2)) < 0.97 * pp;
@@ -950,6 +964,9 @@ int flash_bf16_split_plan(const mx_attn_params& p, int cus, int* full, int* unit
   const Bf16Plan pl = bf16_plan(p, cus);
   *full = pl.full, *units = pl.units, *parts = pl.parts;
   return 0;
+}
+int flash_bf16_unit_queries(const mx_attn_params& p, int cus) {
+  return bf16_plan(p, cus).parts == 1 && use_ks(p, cus) ? 128 : 256;
 }
 
 // Launch the fast path. Preconditions (checked by the caller): D in {64, 72, 128},

@@ -227,3 +227,30 @@ def test_flash_split_plan():
         assert f == 0 and u == ntq * shape[2] and 2 <= s <= 8 and s * 4 <= -(-shape[1] // 64), (shape, f, u, s)
     # the plan depends on the CU count it is given: 1 CU runs every grid whole
     assert flash_attn_split_plan(P(256, 2048, 2), 1) == (2, 0, 1)
+
+
+@pytest.mark.parametrize("Sq,off,H,queries", [
+    # at most one round of 256-query units, and one of 128-query units: always the short ones
+    (333, 0, 32, 128), (1000, 8192, 32, 128), (512, 8192, 64, 128), (2048, 8192, 16, 128),
+    # two rounds of 128-query units: where the units differ in length
+    (2048, 0, 32, 128), (2048, 117, 32, 128), (2048, 2048, 32, 128), (1500, 2048, 32, 128), (1000, 1024, 64, 128),
+    (4096, 4096, 16, 128), (2560, 4096, 16, 128),
+    # and not behind a long cache, where they are nearly alike
+    (2048, 8192, 32, 256), (1500, 8192, 32, 256), (1000, 4096, 64, 256), (2560, 8192, 16, 256),
+    (900, 2300, 48, 256), (1000, 2601, 64, 256),
+    # more than one round of 256-query units; fewer than three key tiles
+    (3000, 0, 32, 256), (100, 0, 32, 256),
+])
+def test_causal_unit_size(Sq, off, H, queries):
+    """Causal calls on 256 CUs: each line was measured with both kernels. Host-side."""
+    from miroxen_amd.attention import flash_attn_unit_queries
+    p = AttnParams(Sq=Sq, Skv=Sq + off, Hq=H, Hkv=H // 4, D=128, causal=1, q_offset=off)
+    assert flash_attn_unit_queries(p, 256) == queries
+
+
+def test_causal_unit_size_extreme_offsets():
+    """No query sees a key; every query sees all of them: no overflow, no division."""
+    from miroxen_amd.attention import flash_attn_unit_queries
+    for off, queries in ((-2**31, 128), (-5000, 128), (2**31 - 1, 256)):
+        p = AttnParams(Sq=2048, Skv=2165, Hq=32, Hkv=8, D=128, causal=1, q_offset=off)
+        assert flash_attn_unit_queries(p, 256) == queries, off

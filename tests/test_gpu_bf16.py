@@ -343,6 +343,8 @@ KS = [
     (385, 640, 24, 12, 64, 0, 0, 5, (0, 0)), (900, 1000, 8, 8, 64, 1, 100, 0, (300, 400)),
     (700, 700, 12, 12, 128, 1, 0, 0, (0, 0)),
     (2100, 2100, 32, 8, 128, 1, 0, 0, (0, 0)), (5600, 5600, 12, 4, 128, 1, 0, 0, (0, 0)),
+    # behind a long cache: 256-query units again, one round of them
+    (900, 3200, 48, 8, 128, 1, 2300, 0, (0, 0)), (1000, 3601, 64, 8, 72, 1, 2601, 5, (64, 128)),
 ]
 
 
