@@ -252,6 +252,12 @@ int mx_quantize_blockscaled(int mode, const void* x, int64_t ldx, int64_t rows, 
 int mx_gemm_blockscaled(int mode, const void* wq, const void* wsf, const float* wamax, const void* xq, const void* xsf,
                         const float* xamax, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, float beta,
                         void* stream);
+/* No counterpart in the reference (a diagnostic query): the output tile that
+ * mx_gemm_blockscaled takes for these sizes on a device with `cus` compute units (cus <= 0:
+ * the current device), *tile_n columns of Y by *tile_m rows, and over how many waves of a
+ * work-group it splits K (*k_waves; 1: K is summed in one chain). Launches nothing. */
+int mx_gemm_blockscaled_tile(int mode, int64_t M, int64_t N, int64_t K, int cus, int* tile_n, int* tile_m,
+                             int* k_waves);
 
 #ifdef __cplusplus
 }

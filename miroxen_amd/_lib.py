@@ -22,6 +22,7 @@ SYMBOLS = (
     "mx_sage_quantize", "mx_sage_attend", "mx_last_error", "mx_version", "mx_head_norm_rope",
     "mx_sage_quantize_norm_rope", "mx_flash_attn_fp8_norm_rope", "mx_sage_quantize_qgroup", "mx_sage_prologue_wait_ticks",
     "mx_qmode_supported", "mx_qdata_bytes", "mx_qscale_bytes", "mx_quantize_blockscaled", "mx_gemm_blockscaled",
+    "mx_gemm_blockscaled_tile",
 )
 
 
@@ -89,6 +90,8 @@ def load():
                                      vp], ctypes.c_int),
         "mx_gemm_blockscaled": ([ctypes.c_int, vp, vp, vp, vp, vp, vp, vp, ctypes.c_int64, ctypes.c_int64,
                                  ctypes.c_int64, ctypes.c_int64, ctypes.c_float, vp], ctypes.c_int),
+        "mx_gemm_blockscaled_tile": ([ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ip,
+                                      ip, ip], ctypes.c_int),
     }
     for name, (args, res) in sig.items():
         fn = getattr(L, name)

@@ -73,3 +73,13 @@ def gemm_blockscaled(m: QMode, W: QMat, X: QMat, Y, ldy: int, M: int, N: int, K:
     _lib.check(_lib.load().mx_gemm_blockscaled(int(m), _addr(W.q), _addr(W.sf), _addr(W.amax), _addr(X.q),
                                                _addr(X.sf), _addr(X.amax), _addr(Y), ldy, M, N, K, beta,
                                                _stream(stream)))
+
+
+def gemm_blockscaled_tile(m: QMode, M: int, N: int, K: int, cus: int = 0) -> tuple:
+    """(tile_n, tile_m, k_waves): the output tile that gemm_blockscaled takes for these sizes
+    on a device with `cus` compute units (0: the current device) and the waves it splits K
+    over; a diagnostic query with no counterpart in the reference."""
+    n, t, w = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+    _lib.check(_lib.load().mx_gemm_blockscaled_tile(int(m), M, N, K, int(cus), ctypes.byref(n), ctypes.byref(t),
+                                                    ctypes.byref(w)))
+    return n.value, t.value, w.value

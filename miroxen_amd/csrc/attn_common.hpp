@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <type_traits>
 #include <utility>
 #include <stdint.h>
@@ -210,6 +211,22 @@ __device__ __forceinline__ uint64_t tile_live(const uint64_t* live, const mx_att
 __device__ __forceinline__ int xcd_remap(int b, int n) {
   const int q = n / 8, r = n % 8, x = b % 8, local = b / 8;
   return x * q + (x < r ? x : r) + local;
+}
+
+// Compute units of device `dev` (0: unknown), asked for once per device; threads that race to
+// fill an entry store the same value. The second form: of the current device, or an MI355X's.
+inline int device_cus(int dev) {
+  static std::atomic<int> cus[64];
+  if (dev < 0 || dev >= 64) return 0;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+    cus[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
+inline int current_cus() {
+  int dev = 0;
+  const int n = hipGetDevice(&dev) == hipSuccess ? device_cus(dev) : 0;
+  return n > 0 ? n : 256;
 }
 
 #ifdef MX_STAMPS

@@ -1021,9 +1021,9 @@ hipError_t launch_mxfp8_quant(const uint16_t* x, int64_t ldx, int64_t rows, int6
 namespace {
 
 // The tile of a GEMM, by its estimated time in us: f0 + rounds (f + a nst), nst K stages of
-// 128 bytes, rounds of 256 CUs x occ work-groups; `alone` replaces a where two work-groups
-// fit a CU and no more than 256 run. The figures are fits to sweeps of M 1 .. 8192, N and K
-// 1024 .. 12288 on an MI355X, operands rotating through 3 buffers (us, best of the others):
+// 128 bytes, rounds of C CUs x occ work-groups; `alone` replaces a where two work-groups
+// fit a CU and no more than C run. The figures are fits to sweeps of M 1 .. 8192, N and K
+// 1024 .. 12288 on an MI355X (C = 256), operands rotating through 3 buffers (us, best of the others):
 //   M     N     K       256 x 256  256 x 128  128 x 128  64 x 64   64 x 64   64 x 32  32 x 32
 //                                                        4 waves   2 waves
 //   1     3072  3072    28.2       17.6       11.9       7.2       8.6       6.2      5.0
@@ -1038,26 +1038,26 @@ namespace {
 // them the time is the latency of K in series, which the K-split tiles divide by their waves.
 enum GemmKind { kG256, kG256x128, kG128, kGk64, kGk64w2, kGk64x32, kGk32, kGKinds };
 struct GemmTile {
-  int tn, tm, occ;
+  int tn, tm, occ, ks;  // ks: waves that K is split over
   double f0, f, a, alone;
 };
 constexpr GemmTile kMxTiles[kGKinds] = {
-    {256, 256, 1, 2.0, 8.0, 1.05, 0}, {256, 128, 1, 0, 7.0, 0.58, 0},      {128, 128, 1, 0, 5.5, 0.39, 0},
-    {64, 64, 1, 1.5, 3.4, 0.175, 0},  {64, 64, 2, 1.1, 3.9, 0.325, 0.226}, {64, 32, 1, 1.2, 3.0, 0.13, 0},
-    {32, 32, 2, 0.5, 2.8, 0.20, 0.095}};
-GemmKind gemm_plan(const GemmTile (&tiles)[kGKinds], int M, int N, int nst) {
+    {256, 256, 1, 1, 2.0, 8.0, 1.05, 0}, {256, 128, 1, 1, 0, 7.0, 0.58, 0},      {128, 128, 1, 1, 0, 5.5, 0.39, 0},
+    {64, 64, 1, 4, 1.5, 3.4, 0.175, 0},  {64, 64, 2, 2, 1.1, 3.9, 0.325, 0.226}, {64, 32, 1, 4, 1.2, 3.0, 0.13, 0},
+    {32, 32, 2, 4, 0.5, 2.8, 0.20, 0.095}};
+GemmKind gemm_plan(const GemmTile (&tiles)[kGKinds], int M, int N, int nst, int C) {
   int best = 0;
   double bt = 0;
   for (int k = 0; k < kGKinds; ++k) {
     const GemmTile& t = tiles[k];
     const int64_t n = int64_t((N + t.tn - 1) / t.tn) * ((M + t.tm - 1) / t.tm);
-    const double rounds = double((n + 256 * t.occ - 1) / (256 * t.occ));
-    const double us = t.f0 + rounds * (t.f + nst * (t.occ == 2 && n <= 256 ? t.alone : t.a));
+    const double rounds = double((n + int64_t(C) * t.occ - 1) / (int64_t(C) * t.occ));
+    const double us = t.f0 + rounds * (t.f + nst * (t.occ == 2 && n <= C ? t.alone : t.a));
     if (k == 0 || us < bt) best = k, bt = us;
   }
   return GemmKind(best);
 }
-GemmKind mxfp8_plan(int M, int N, int K) { return gemm_plan(kMxTiles, M, N, (K + kStage - 1) / kStage); }
+GemmKind mxfp8_plan(int M, int N, int K, int C) { return gemm_plan(kMxTiles, M, N, (K + kStage - 1) / kStage, C); }
 
 }  // namespace
 
@@ -1065,7 +1065,7 @@ GemmKind mxfp8_plan(int M, int N, int K) { return gemm_plan(kMxTiles, M, N, (K +
 // same for M; beta 0 or 1.
 hipError_t launch_mxfp8_gemm(const uint8_t* wq, const uint8_t* wsf, const uint8_t* xq, const uint8_t* xsf,
                              uint16_t* y, int64_t ldy, int M, int N, int K, int beta, hipStream_t s) {
-  const GemmKind kind = mxfp8_plan(M, N, K);
+  const GemmKind kind = mxfp8_plan(M, N, K, current_cus());
   const int tn = kMxTiles[kind].tn, tm = kMxTiles[kind].tm, ntn = (N + tn - 1) / tn, ntm = (M + tm - 1) / tm;
   const int64_t blocks = int64_t(ntn) * ntm;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
@@ -1073,17 +1073,17 @@ hipError_t launch_mxfp8_gemm(const uint8_t* wq, const uint8_t* wsf, const uint8_
   auto tiles = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, wq, wsf, xq, xsf, y, ldy, M, N, K, beta, ntn, ntm);
   };
-  auto ksplit = [&](auto kern, int ks) {
-    hipLaunchKernelGGL(kern, grid, dim3(64 * ks), 0, s, wq, wsf, (const float*)nullptr, xq, xsf, (const float*)nullptr,
+  auto ksplit = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kMxTiles[kind].ks), 0, s, wq, wsf, (const float*)nullptr, xq, xsf, (const float*)nullptr,
                        y, ldy, M, N, K, beta, ntm);
   };
   switch (kind) {
     case kG256x128: tiles(mxfp8_gemm<4, 2, 3>); break;
     case kG128: tiles(mxfp8_gemm<2, 2, 4>); break;
-    case kGk64: ksplit(gemm_ksplit<false, 2, 2, 4, 2>, 4); break;
-    case kGk64w2: ksplit(gemm_ksplit<false, 2, 2, 2, 2>, 2); break;
-    case kGk64x32: ksplit(gemm_ksplit<false, 2, 1, 4, 3>, 4); break;
-    case kGk32: ksplit(gemm_ksplit<false, 1, 1, 4, 2>, 4); break;
+    case kGk64: ksplit(gemm_ksplit<false, 2, 2, 4, 2>); break;
+    case kGk64w2: ksplit(gemm_ksplit<false, 2, 2, 2, 2>); break;
+    case kGk64x32: ksplit(gemm_ksplit<false, 2, 1, 4, 3>); break;
+    case kGk32: ksplit(gemm_ksplit<false, 1, 1, 4, 2>); break;
     default: tiles(mxfp8_gemm<4, 4, 2>); break;
   }
   return hipGetLastError();
@@ -1121,19 +1121,26 @@ namespace {
 //   2048  3072  3072    56         39         43         60        50        90       76
 //   4096  3072  12288   227        283        262        350       337       461      547
 constexpr GemmTile kF4Tiles[kGKinds] = {
-    {256, 256, 1, 0, 8.0, 3.9, 0},   {256, 128, 1, 0, 7.7, 2.4, 0},    {128, 128, 2, 0, 4.4, 3.2, 1.6},
-    {64, 64, 1, 1.0, 4.5, 0.45, 0},  {64, 64, 2, 1.0, 4.2, 1.02, 0.87}, {64, 32, 1, 0.9, 3.7, 0.32, 0},
-    {32, 32, 2, 0.5, 2.7, 0.53, 0.25}};
-GemmKind nvfp4_plan(int M, int N, int K) { return gemm_plan(kF4Tiles, M, N, (K / 2 + kStage - 1) / kStage); }
+    {256, 256, 1, 1, 0, 8.0, 3.9, 0},   {256, 128, 1, 1, 0, 7.7, 2.4, 0},    {128, 128, 2, 1, 0, 4.4, 3.2, 1.6},
+    {64, 64, 1, 4, 1.0, 4.5, 0.45, 0},  {64, 64, 2, 2, 1.0, 4.2, 1.02, 0.87}, {64, 32, 1, 4, 0.9, 3.7, 0.32, 0},
+    {32, 32, 2, 4, 0.5, 2.7, 0.53, 0.25}};
+GemmKind nvfp4_plan(int M, int N, int K, int C) {
+  return gemm_plan(kF4Tiles, M, N, (K / 2 + kStage - 1) / kStage, C);
+}
 
 }  // namespace
+
+void gemm_blockscaled_tile(bool f4, int M, int N, int K, int cus, int* tile_n, int* tile_m, int* k_waves) {
+  const GemmTile& t = f4 ? kF4Tiles[nvfp4_plan(M, N, K, cus)] : kMxTiles[mxfp8_plan(M, N, K, cus)];
+  *tile_n = t.tn, *tile_m = t.tm, *k_waves = t.ks;
+}
 
 // Preconditions (checked by the caller): K % 32 == 0, (N + 255) / 256 * 256 * K / 2 < 2^31,
 // same for M; beta 0 or 1; the amax pointers are device floats written by the quantizer.
 hipError_t launch_nvfp4_gemm(const uint8_t* wq, const uint8_t* wsf, const float* wamax, const uint8_t* xq,
                              const uint8_t* xsf, const float* xamax, uint16_t* y, int64_t ldy, int M, int N, int K,
                              int beta, hipStream_t s) {
-  const GemmKind kind = nvfp4_plan(M, N, K);
+  const GemmKind kind = nvfp4_plan(M, N, K, current_cus());
   const int tn = kF4Tiles[kind].tn, tm = kF4Tiles[kind].tm, ntn = (N + tn - 1) / tn, ntm = (M + tm - 1) / tm;
   const int64_t blocks = int64_t(ntn) * ntm;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
@@ -1141,16 +1148,16 @@ hipError_t launch_nvfp4_gemm(const uint8_t* wq, const uint8_t* wsf, const float*
   auto tiles = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntn, ntm);
   };
-  auto ksplit = [&](auto kern, int ks) {
-    hipLaunchKernelGGL(kern, grid, dim3(64 * ks), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntm);
+  auto ksplit = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kF4Tiles[kind].ks), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntm);
   };
   switch (kind) {
     case kG256x128: tiles(nvfp4_gemm<4, 2>); break;
     case kG128: tiles(nvfp4_gemm<2, 2>); break;
-    case kGk64: ksplit(gemm_ksplit<true, 2, 2, 4, 2>, 4); break;
-    case kGk64w2: ksplit(gemm_ksplit<true, 2, 2, 2, 2>, 2); break;
-    case kGk64x32: ksplit(gemm_ksplit<true, 2, 1, 4, 3>, 4); break;
-    case kGk32: ksplit(gemm_ksplit<true, 1, 1, 4, 2>, 4); break;
+    case kGk64: ksplit(gemm_ksplit<true, 2, 2, 4, 2>); break;
+    case kGk64w2: ksplit(gemm_ksplit<true, 2, 2, 2, 2>); break;
+    case kGk64x32: ksplit(gemm_ksplit<true, 2, 1, 4, 3>); break;
+    case kGk32: ksplit(gemm_ksplit<true, 1, 1, 4, 2>); break;
     default: tiles(nvfp4_gemm<4, 4>); break;
   }
   return hipGetLastError();

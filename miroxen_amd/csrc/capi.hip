@@ -37,6 +37,7 @@ hipError_t launch_mxfp8_gemm(const uint8_t*, const uint8_t*, const uint8_t*, con
 hipError_t launch_nvfp4_quant(const uint16_t*, int64_t, int64_t, int64_t, uint8_t*, uint8_t*, float*, hipStream_t);
 hipError_t launch_nvfp4_gemm(const uint8_t*, const uint8_t*, const float*, const uint8_t*, const uint8_t*, const float*,
                              uint16_t*, int64_t, int, int, int, int, hipStream_t);
+void gemm_blockscaled_tile(bool f4, int M, int N, int K, int cus, int* tile_n, int* tile_m, int* k_waves);
 }  // namespace mxa
 
 namespace {
@@ -507,6 +508,25 @@ int mx_quantize_blockscaled(int mode, const void* x, int64_t ldx, int64_t rows, 
                     "quantize_blockscaled");
 }
 
+// 32-bit buffer offsets within a 256-row tile's operand, and int grid coordinates.
+static bool gemm_fits(int64_t M, int64_t N, int64_t K) {
+  return (N + 255) / 256 * 256 * K < (int64_t(1) << 31) && (M + 255) / 256 * 256 * K < (int64_t(1) << 31) &&
+         M <= 0x7fffffff && N <= 0x7fffffff;
+}
+
+int mx_gemm_blockscaled_tile(int mode, int64_t M, int64_t N, int64_t K, int cus, int* tile_n, int* tile_m,
+                             int* k_waves) {
+  if (!tile_n || !tile_m || !k_waves) return fail(MX_E_INVALID, "gemm_blockscaled_tile: null argument");
+  if (mode != MX_QMODE_MXFP8 && mode != MX_QMODE_NVFP4)
+    return fail(MX_E_INVALID, "gemm_blockscaled_tile: mode %d is not a quantized mode", mode);
+  if (M <= 0 || N <= 0 || K <= 0 || K % 32) return fail(MX_E_INVALID, "gemm_blockscaled_tile: bad shape");
+  if (!gemm_fits(M, N, K)) return fail(MX_E_UNSUPPORTED, "gemm_blockscaled_tile: matrix too large for 32-bit offsets");
+  const int rc = query_cus(&cus, "gemm_blockscaled_tile");
+  if (rc != MX_OK) return rc;
+  mxa::gemm_blockscaled_tile(mode == MX_QMODE_NVFP4, int(M), int(N), int(K), cus, tile_n, tile_m, k_waves);
+  return MX_OK;
+}
+
 int mx_gemm_blockscaled(int mode, const void* wq, const void* wsf, const float* wamax, const void* xq, const void* xsf,
                         const float* xamax, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, float beta,
                         void* stream) {
@@ -521,9 +541,7 @@ int mx_gemm_blockscaled(int mode, const void* wq, const void* wsf, const float* 
       !aligned(xq, 16) || !aligned(wsf, 4) || !aligned(xsf, 4) || !aligned(y, 2))
     return fail(MX_E_INVALID, "gemm_blockscaled: bad arguments (M=%lld N=%lld K=%lld)", (long long)M, (long long)N,
                 (long long)K);
-  // 32-bit buffer offsets within a 256-row tile's operand, and int grid coordinates
-  if ((N + 255) / 256 * 256 * K >= (int64_t(1) << 31) || (M + 255) / 256 * 256 * K >= (int64_t(1) << 31) ||
-      M > 0x7fffffff || N > 0x7fffffff)
+  if (!gemm_fits(M, N, K))
     return fail(MX_E_UNSUPPORTED, "gemm_blockscaled: matrix too large for 32-bit offsets");
   if (mode == MX_QMODE_NVFP4)
     return hip_status(mxa::launch_nvfp4_gemm(static_cast<const uint8_t*>(wq), static_cast<const uint8_t*>(wsf), wamax,

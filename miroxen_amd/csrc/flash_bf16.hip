@@ -27,7 +27,6 @@
 //    than all waves in lockstep. Within an MFMA phase, sched_group_barrier keeps
 //    LDS operand reads a few MFMAs ahead of use (kKPrefetch / kVPrefetch).
 //  * Work-groups are remapped so one head's query tiles share an XCD (and its L2).
-#include <atomic>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -921,8 +920,7 @@ Bf16Plan bf16_plan(const mx_attn_params& p, int C) {
   return pl;
 }
 
-// Per-device state of the split. cus is read without a lock (every thread that races
-// to fill it stores the same value). The region's address and the ordering event are
+// Per-device state of the split. The region's address and the ordering event are
 // set up once per device, on the first call that splits; after that a split call
 // takes the device's mutex only to order itself after the previous split call
 // (stream wait on the event, launches, event record), so calls on different streams
@@ -930,7 +928,6 @@ Bf16Plan bf16_plan(const mx_attn_params& p, int C) {
 // causal calls, calls under stream capture) take no lock and touch no shared state.
 constexpr int kMaxDev = 64;
 struct SplitDevice {
-  std::atomic<int> cus{0};
   std::once_flag once;
   hipError_t setup = hipSuccess;
   void* region = nullptr;
@@ -938,13 +935,6 @@ struct SplitDevice {
   std::mutex mu;
 };
 SplitDevice g_split[kMaxDev];
-
-int device_cus(SplitDevice& R, int dev) {
-  int n = R.cus.load(std::memory_order_relaxed);
-  if (n == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-    R.cus.store(n, std::memory_order_relaxed);
-  return n;
-}
 
 hipError_t split_setup(SplitDevice& R) {
   std::call_once(R.once, [&R] {
@@ -991,7 +981,7 @@ hipError_t launch_flash_bf16(const uint16_t* q, const uint16_t* k, const uint16_
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < kMaxDev) {
       R = &g_split[dev];
-      const int cus = device_cus(*R, dev);
+      const int cus = device_cus(dev);
       pl = bf16_plan(p, cus);  // (causal calls never split)
       ks = pl.parts == 1 && use_ks(p, cus);
     }

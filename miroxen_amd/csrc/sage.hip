@@ -1596,13 +1596,11 @@ uint64_t next_epoch() {
 }
 
 // Work-groups per (head, 256-token block) of the one-pass prologue: K and V apart while every
-// half still gets a CU of its own (256). Call us, one / two: 24 heads x 256 keys 21.1 / 19.3,
+// half still gets a CU of its own. On 256 CUs, call us, one / two: 24 heads x 256 keys 21.1 / 19.3,
 // x 600 26.7 / 25.3, x 1088 (120 blocks) 33.0 / 31.3, 8 x 4096 (128) 64.6 / 62.5; with norm/RoPE
 // 25.4 / 22.4, 32.2 / 29.1, 39.9 / 36.3, 70.2 / 66.6. Beyond, the halves queue for the same
 // CUs and gain nothing or lose: 24 x 1500 (144) 49.5 / 49.5 and 55.3 / 56.5, x 4352 181 / 186.
-int fused_sides(int64_t blocks) {
-  return blocks <= 128 ? 2 : 1;
-}
+int fused_sides(int64_t blocks, int cus) { return 2 * blocks <= cus ? 2 : 1; }
 
 mx_sage_layout sage_layout(const mx_attn_params& p) {
   mx_sage_layout L{};
@@ -1662,7 +1660,7 @@ hipError_t sage_quantize_d(const uint16_t* q, const uint16_t* k, const uint16_t*
   decltype(&prep_stats_q<D, -1, 16>) stats;
   decltype(&prep_kv_quant<D, -1>) kvq;
   decltype(&prep_kv_fused<D, -1, 1>) fused;
-  const int sides = fused_sides(int64_t(p.Hkv) * nb);
+  const int sides = fused_sides(int64_t(p.Hkv) * nb, current_cus());
   auto pick = [&](auto nrm) {
     constexpr int N = decltype(nrm)::value;
     return sides == 2 ? prep_kv_fused<D, N, 2> : prep_kv_fused<D, N, 1>;

@@ -254,3 +254,33 @@ def test_causal_unit_size_extreme_offsets():
     for off, queries in ((-2**31, 128), (-5000, 128), (2**31 - 1, 256)):
         p = AttnParams(Sq=2048, Skv=2165, Hq=32, Hkv=8, D=128, causal=1, q_offset=off)
         assert flash_attn_unit_queries(p, 256) == queries, off
+
+
+def test_gemm_tile_of_the_shapes_tested_on_the_device():
+    """The shapes by which the GPU tests reach every output tile and every remainder of its
+    stage ring, on 256 CUs. Host-side."""
+    from miroxen_amd.blockscale import QMode, gemm_blockscaled_tile
+    from tests.test_gpu_blockscale import KSPLIT, KSPLIT4, RING, TILES, TILES4
+    for mode, shapes in ((QMode.MXFP8, TILES + KSPLIT), (QMode.NVFP4, TILES4 + KSPLIT4)):
+        for M, N, K, *_, tile in shapes:
+            assert gemm_blockscaled_tile(mode, M, N, K, 256) == tile, (mode, M, N, K)
+        assert len({c[-1] for c in shapes}) == 7
+    for M, N, K, tile in RING:
+        assert gemm_blockscaled_tile(QMode.MXFP8, M, N, K, 256) == tile, (M, N, K)
+
+
+def test_gemm_tile_follows_the_cus():
+    """Fewer CUs fill up with fewer tiles: a GEMM that splits K on 256 of them takes whole
+    large tiles on a part of the chip. Host-side."""
+    from miroxen_amd.blockscale import QMode, gemm_blockscaled_tile
+    tile = lambda mode, cus: gemm_blockscaled_tile(mode, 256, 3072, 3072, cus)
+    assert [tile(QMode.MXFP8, c) for c in (256, 128, 64, 32)] == [
+        (64, 64, 4), (64, 64, 2), (128, 128, 1), (256, 128, 1)]
+    for mode in (QMode.MXFP8, QMode.NVFP4):
+        assert gemm_blockscaled_tile(mode, 8192, 12288, 4096, 256) == (256, 256, 1)
+        assert tile(mode, 256)[2] > 1 and tile(mode, 32)[2] == 1
+    for bad in ((0, 64, 64), (64, 64, 40), (1 << 20, 64, 4096)):
+        with pytest.raises(RuntimeError):
+            gemm_blockscaled_tile(QMode.MXFP8, *bad, 256)
+    with pytest.raises(RuntimeError):
+        gemm_blockscaled_tile(QMode.BF16, 64, 64, 64, 256)

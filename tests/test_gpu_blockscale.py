@@ -8,8 +8,8 @@ import pytest
 import torch
 
 import oracle
-from miroxen_amd.blockscale import (QMat, QMode, gemm_blockscaled, qdata_bytes, qmode_supported, qscale_bytes,
-                                    quantize_blockscaled)
+from miroxen_amd.blockscale import (QMat, QMode, gemm_blockscaled, gemm_blockscaled_tile, qdata_bytes,
+                                    qmode_supported, qscale_bytes, quantize_blockscaled)
 
 pytestmark = pytest.mark.gpu
 
@@ -147,15 +147,24 @@ def test_gemm_full_size_sampled_rows(cuda):
 # K split over four and two waves, 128 x 128, 256 x 128, 256 x 256), each with ragged rows and
 # columns and a K that is no whole number of 128-byte stages (nor of turns of the stage
 # ring), padded, odd (element-wise stores) and accumulating outputs among them.
-TILES = [
-    (33, 8130, 160, 1, 0.0), (45, 6010, 1120, 6, 1.0), (40, 9000, 96, 0, 0.0), (40, 5000, 2080, 2, 1.0),
-    (200, 5000, 608, 0, 0.0), (257, 8130, 608, 1, 1.0), (700, 6200, 736, 4, 0.0), (1500, 6100, 352, 3, 1.0),
+TILES = [  # M, N, K, padding of a row of Y, beta; the tile as gemm_blockscaled_tile reports it
+    (33, 8130, 160, 1, 0.0, (32, 32, 4)), (45, 6010, 1120, 6, 1.0, (32, 32, 4)), (40, 9000, 96, 0, 0.0, (64, 64, 4)),
+    (40, 5000, 2080, 2, 1.0, (64, 32, 4)), (200, 5000, 608, 0, 0.0, (64, 64, 2)),
+    (257, 8130, 608, 1, 1.0, (128, 128, 1)), (700, 6200, 736, 4, 0.0, (256, 128, 1)),
+    (1500, 6100, 352, 3, 1.0, (256, 256, 1)),
 ]
+# The waves of a K-split tile take every fourth (second) stage, each in its own ring of two or
+# three slots: every remainder of a wave's stages modulo its slots, also unlike ones in a group.
+KSPLIT = [(200, 1000, 128 * st, 0, 0.0, (32, 32, 4)) for st in (4, 5, 7, 12)] + [
+    (40, 5000, 128 * st, 0, 0.0, (64, 32, 4)) for st in (13, 16, 18, 22, 24)] + [
+    (70, 5500, 128 * st, 0, 0.0, (64, 64, 4)) for st in (3, 8, 11)] + [
+    (150, 5500, 128 * st, 0, 0.0, (64, 64, 2)) for st in (1, 4, 5, 6)]
 
 
-def _sampled_rows_match(mode, M, N, K, pad, beta, cuda):
-    """Output rows around every tile edge against the oracle GEMM of those rows."""
+def _sampled_rows_match(mode, M, N, K, pad, beta, tile, cuda):
+    """Output rows around the tile edges and one in every 32 against the oracle GEMM of those rows."""
     print(f"{mode.name} gemm tiles M={M} N={N} K={K} pad={pad} beta={beta}", flush=True)
+    assert gemm_blockscaled_tile(mode, M, N, K) == tile
     rng = np.random.default_rng(M + 3 * N + K)
     xb = oracle.f32_to_bf16((rng.standard_normal((M, K)) * 2).astype(np.float32))
     wb = oracle.f32_to_bf16((rng.standard_normal((N, K)) * 0.05).astype(np.float32))
@@ -167,7 +176,8 @@ def _sampled_rows_match(mode, M, N, K, pad, beta, cuda):
     gemm_blockscaled(mode, QMat(*W), QMat(*X), y, N + pad, M, N, K, beta)
     torch.cuda.synchronize()
     got = oracle.bf16_to_f32(y.cpu().numpy().view(np.uint16)).astype(np.float64)
-    rows = np.array(sorted({r for t in (0, 32, 64, 128, 192, 256, M) for r in (t - 1, t) if 0 <= r < M}))
+    rows = {r for t in (0, 32, 64, 128, 192, 256, M) for r in (t - 1, t) if 0 <= r < M}
+    rows = np.array(sorted(rows | {min(M - 1, t + t // 32 % 32) for t in range(0, M, 32)}))
     if mode == QMode.MXFP8:
         want = oracle.gemm_mxfp8(*oracle.mxfp8_quantize(wb, N, K), *oracle.mxfp8_quantize(xb[rows], len(rows), K),
                                  len(rows), N, K)
@@ -182,18 +192,21 @@ def _sampled_rows_match(mode, M, N, K, pad, beta, cuda):
     np.testing.assert_array_equal(got[:, N:], old[:, N:])  # columns past N untouched
 
 
-@pytest.mark.parametrize("M,N,K,pad,beta", TILES)
-def test_gemm_tile_kinds(cuda, M, N, K, pad, beta):
-    _sampled_rows_match(QMode.MXFP8, M, N, K, pad, beta, cuda)
+@pytest.mark.parametrize("M,N,K,pad,beta,tile", TILES + KSPLIT)
+def test_gemm_tile_kinds(cuda, M, N, K, pad, beta, tile):
+    _sampled_rows_match(QMode.MXFP8, M, N, K, pad, beta, tile, cuda)
 
 
 # Every remainder of the K stages modulo the ring depth of the 256 x 128 (3 slots) and 128 x 128
 # (4 slots) tiles, behind at least one whole turn of the ring.
-@pytest.mark.parametrize("M,N,K", [(700, 5500, 128 * st - pad) for st, pad in ((7, 0), (8, 32), (9, 96))] +
-                         [(300, 7000, 128 * st - pad) for st, pad in ((7, 0), (8, 32), (9, 64), (10, 0), (11, 96))] +
-                         [(512, 5120, 896), (512, 5120, 3456)])
-def test_gemm_ring_remainders(cuda, M, N, K):
-    _sampled_rows_match(QMode.MXFP8, M, N, K, 0, 0.0, cuda)
+RING = [(700, 5500, 128 * st - pad, (256, 128, 1)) for st, pad in ((7, 0), (8, 32), (9, 96))] + [
+    (300, 7000, 128 * st - pad, (128, 128, 1)) for st, pad in ((7, 0), (8, 32), (9, 64), (10, 0), (11, 96))] + [
+    (512, 5120, 896, (128, 128, 1)), (512, 5120, 3456, (128, 128, 1))]
+
+
+@pytest.mark.parametrize("M,N,K,tile", RING)
+def test_gemm_ring_remainders(cuda, M, N, K, tile):
+    _sampled_rows_match(QMode.MXFP8, M, N, K, 0, 0.0, tile, cuda)
 
 
 # ---------------- NVFP4 (reference blockscale.cu NVFP4 branch) ----------------
@@ -262,14 +275,19 @@ def test_nvfp4_gemm_matches_oracle(cuda, M, N, K, beta):
 
 # The same choice for NVFP4 (stages of 256 values).
 TILES4 = [
-    (33, 8130, 288, 1, 0.0), (40, 5000, 2080, 2, 1.0), (70, 6000, 1056, 0, 0.0), (300, 4000, 1312, 6, 1.0),
-    (257, 8130, 1120, 1, 1.0), (700, 6200, 1312, 4, 0.0), (1500, 6100, 608, 3, 1.0),
+    (33, 8130, 288, 1, 0.0, (32, 32, 4)), (40, 5000, 2080, 2, 1.0, (64, 32, 4)), (70, 6000, 1056, 0, 0.0, (64, 64, 4)),
+    (300, 4000, 1312, 6, 1.0, (64, 64, 2)), (257, 8130, 1120, 1, 1.0, (128, 128, 1)),
+    (700, 6200, 1312, 4, 0.0, (256, 128, 1)), (1500, 6100, 608, 3, 1.0, (256, 256, 1)),
 ]
+KSPLIT4 = [(200, 1000, 256 * st, 0, 0.0, (32, 32, 4)) for st in (4, 5, 7, 12)] + [
+    (40, 5000, 256 * st, 0, 0.0, (64, 32, 4)) for st in (8, 13, 16, 18)] + [
+    (70, 5500, 256 * st, 0, 0.0, (64, 64, 4)) for st in (3, 8, 11)] + [
+    (150, 5500, 256 * st, 0, 0.0, (64, 64, 2)) for st in (3, 4, 5, 6)]
 
 
-@pytest.mark.parametrize("M,N,K,pad,beta", TILES4)
-def test_nvfp4_gemm_tile_kinds(cuda, M, N, K, pad, beta):
-    _sampled_rows_match(QMode.NVFP4, M, N, K, pad, beta, cuda)
+@pytest.mark.parametrize("M,N,K,pad,beta,tile", TILES4 + KSPLIT4)
+def test_nvfp4_gemm_tile_kinds(cuda, M, N, K, pad, beta, tile):
+    _sampled_rows_match(QMode.NVFP4, M, N, K, pad, beta, tile, cuda)
 
 
 @pytest.mark.parametrize("M,N,K", [(300, 512, 1024), (129, 384, 4160)])
