@@ -34,10 +34,8 @@ namespace mxa {
 namespace {
 
 constexpr int kMxBlock = 32;       // K values per UE8M0 scale
-constexpr int kTile = 256;         // n and m per work-group
 constexpr int kStage = 128;        // K bytes per LDS stage
-constexpr int kStageB = kTile * kStage;  // 32 KB per operand per stage
-constexpr int kGroupM = 4;               // tile rows per launch-order group
+constexpr int kGroupM = 4;         // tile rows per launch-order group
 
 __host__ __device__ inline int64_t pad_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
@@ -128,13 +126,6 @@ template <int NV>
 __device__ __forceinline__ void dma_op(__amdgpu_buffer_rsrc_t rs, const OpAddr<NV>& a, int jj, uint32_t past, int k0,
                                        unsigned char* dst, int wave) {
   buf2lds16(rs, a.vo[jj] | past, uint32_t(k0), (MXA_LDS void*)(dst + (4 * jj + wave) * 1024));
-}
-template <int NV>
-__device__ __forceinline__ void dma_stage(__amdgpu_buffer_rsrc_t rs, const OpAddr<NV>& a, int64_t K, int k0,
-                                          unsigned char* dst, int wave) {
-  const uint32_t past = past_k(a, K, k0);
-#pragma unroll
-  for (int jj = 0; jj < NV; ++jj) dma_op(rs, a, jj, past, k0, dst, wave);
 }
 
 // Epilogue through LDS: the TN x TM = 64 NI x 64 NJ bf16 Y tile (row m = 128 NI bytes of

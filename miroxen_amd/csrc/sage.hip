@@ -376,7 +376,8 @@ __global__ void __launch_bounds__(256) prep_kv_quant(const uint16_t* __restrict_
 //
 // Waiting: work-groups are dispatched in index order and a head's blocks are
 // consecutive, so a head's blocks all get a slot while earlier heads drain (a head
-// holds at most kFoldNb work-groups). The wait is bounded all the same: after
+// holds SIDES nb work-groups, nb <= kFoldNb; with SIDES = 2 all heads together hold no
+// more than the device has CUs). The wait is bounded all the same: after
 // kFusedWaitTicks of the 100 MHz chip clock a work-group stops waiting and computes
 // every partial whose flag it has not seen from K and V in memory (the same bytes
 // the missing block would write), so the kernel ends whatever the dispatch order.
