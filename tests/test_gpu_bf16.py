@@ -202,6 +202,35 @@ def test_mask_bitmap_paths(cuda, Skv):
     assert cosine(got, want) >= 0.9999 and max_abs(got, want) <= 2e-2
 
 
+@pytest.mark.parametrize("Sq,H,Skv,D,causal", [
+    (40, 2, 1, 128, 0), (40, 2, 3, 64, 0), (300, 24, 66, 128, 0), (300, 24, 67, 72, 0), (130, 24, 257, 128, 0),
+    (500, 32, 1022, 128, 1), (300, 8, 1025, 128, 0), (256, 2, 2047, 64, 0), (256, 3, 17 * 1024 + 2, 128, 0),
+])
+def test_mask_of_a_partial_last_word(cuda, Sq, H, Skv, D, causal):
+    """Masks of a length that is no multiple of four: the last keys count. Three of four
+    keys are padding, so that each of the last ones weighs in the result; the 16-byte path
+    and the byte path (odd mask address) give the same bits, whatever follows the mask."""
+    print(f"partial last word Sq={Sq} H={H} Skv={Skv} D={D} causal={causal}", flush=True)
+    q, k, v, *_ = _make(Sq, Skv, H, H, D, 0, 1.0, Skv, cuda)
+    g = torch.Generator().manual_seed(Skv)
+    mask = (torch.rand(Skv, generator=g) < 0.25).to(torch.uint8) * 3
+    mask[Skv & ~3:] = 1
+    outs = []
+    for off in (0, 1):
+        m = torch.full((Skv + 64,), 1, dtype=torch.uint8, device=cuda)
+        m[off:off + Skv] = mask.to(cuda)
+        p = AttnParams(Sq=Sq, Skv=Skv, Hq=H, Hkv=H, D=D, causal=causal, q_offset=Skv - Sq if causal else 0,
+                       kv_valid=m[off:off + Skv])
+        outs.append(_run(flash_attn, q, k, v, p, Sq, H * D)[0].clone())
+    rows = sorted(set(range(0, Sq, max(1, Sq // 23))) | {Sq - 1})
+    want = oracle.attention_f64(_bits(q), _bits(k), _bits(v), Sq, Skv, H, H, D, 0.0, causal, Skv - Sq if causal else 0,
+                                kv_valid=mask.numpy(), rows=np.array(rows, np.int32)).reshape(len(rows), -1)
+    for o in outs:
+        ok, err, tol, rr = reference_gate(_f32(o[rows]), want)
+        assert ok, f"max_abs={err} limit={tol} rel_rms={rr}"
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 def test_all_masked_and_deterministic(cuda):
     S, H = 300, 2
     q, k, v, *_ = _make(S, S, H, H, 128, 0, 1.0, 5, cuda)
