@@ -810,7 +810,8 @@ gemm_ksplit(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, con
             uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K, int beta, int ntm) {
   constexpr int TN = 32 * NI, TM = 32 * NJ, SA = TN * kStage, ST = (TN + TM) * kStage;
   constexpr int NSC = F4 ? 4 : 1;                       // scale words per row block and stage
-  constexpr int OPS = 4 * (NI + NJ) + 2 * NSC;          // vector-memory operations per stage
+  constexpr int DMA = 4 * (NI + NJ);                    // LDS-DMA operations per stage
+  constexpr int OPS = DMA + 2 * NSC;                    // with the scale loads
   constexpr int RED = NI * NJ * 4096;                   // bytes of one wave's partial tile
   static_assert((NB - 1) * OPS < 64, "the wait counter has 6 bits");
   __shared__ __align__(16) unsigned char lds[KS * NB * ST > KS * RED ? KS * NB * ST : KS * RED];
@@ -867,9 +868,11 @@ gemm_ksplit(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, con
   const int x = (n >> 1) & 7;
   const int cnt = (nst - wave + KS - 1) / KS;  // this wave's stages (wave < KS; may be 0)
   static_for<NB>([&](auto s) __attribute__((always_inline)) { issue(decltype(s)::value, s); });
-  auto body = [&](int i, auto sc) __attribute__((always_inline)) {
+  // (rest: the stages behind the whole turns, where the compiler deletes scale loads that nothing
+  // uses: only the DMA ops of the younger stages are counted)
+  auto body = [&](int i, auto sc, auto rest) __attribute__((always_inline)) {
     constexpr int s = decltype(sc)::value;
-    wait_vm_n<(NB - 1) * OPS>();
+    wait_vm_n<(NB - 1) * (decltype(rest)::value ? DMA : OPS)>();
     const unsigned char* d = ring + s * ST + n * kStage;
     // this half's 16-byte chunks of a row: 2 r + h
     i32x4 av[NI][4], bv[NJ][4];
@@ -947,9 +950,9 @@ gemm_ksplit(const uint8_t* __restrict__ wq, const uint8_t* __restrict__ wsf, con
   // whole turns of the ring, then the rest (see mxfp8_gemm)
   int i = 0;
   for (; i + NB <= cnt; i += NB)
-    static_for<NB>([&](auto s) __attribute__((always_inline)) { body(i + decltype(s)::value, s); });
+    static_for<NB>([&](auto s) __attribute__((always_inline)) { body(i + decltype(s)::value, s, std::false_type{}); });
   static_for<NB - 1>([&](auto s) __attribute__((always_inline)) {
-    if (i + decltype(s)::value < cnt) body(i + decltype(s)::value, s);
+    if (i + decltype(s)::value < cnt) body(i + decltype(s)::value, s, std::true_type{});
   });
   wait_vm();        // no LDS-DMA may land in what the reduction writes
   __syncthreads();  // every wave is done with the rings
@@ -1065,8 +1068,8 @@ hipError_t launch_mxfp8_gemm(const uint8_t* wq, const uint8_t* wsf, const uint8_
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, wq, wsf, xq, xsf, y, ldy, M, N, K, beta, ntn, ntm);
   };
   auto ksplit = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(64 * kMxTiles[kind].ks), 0, s, wq, wsf, (const float*)nullptr, xq, xsf, (const float*)nullptr,
-                       y, ldy, M, N, K, beta, ntm);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kMxTiles[kind].ks), 0, s, wq, wsf, (const float*)nullptr, xq, xsf,
+                       (const float*)nullptr, y, ldy, M, N, K, beta, ntm);
   };
   switch (kind) {
     case kG256x128: tiles(mxfp8_gemm<4, 2, 3>); break;
@@ -1140,7 +1143,8 @@ hipError_t launch_nvfp4_gemm(const uint8_t* wq, const uint8_t* wsf, const float*
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntn, ntm);
   };
   auto ksplit = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(64 * kF4Tiles[kind].ks), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K, beta, ntm);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kF4Tiles[kind].ks), 0, s, wq, wsf, wamax, xq, xsf, xamax, y, ldy, M, N, K,
+                       beta, ntm);
   };
   switch (kind) {
     case kG256x128: tiles(nvfp4_gemm<4, 2>); break;
